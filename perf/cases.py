@@ -413,7 +413,7 @@ def exact(case, seed):
         if case["mode"] == "unscaled":
             return _mm(_e4m3_nearest(x), w)
         amax = x.abs().amax(-1, keepdim=True)
-        codes = (x * (448.0 / amax)).clamp(-448.0, 448.0).to(torch.float8_e4m3fn)
+        codes = (x * (torch.full_like(amax, 448.0) / amax)).clamp(-448.0, 448.0).to(torch.float8_e4m3fn)
         return _mm(codes.double() * (amax.double() / 448.0), w)
     if kind == "marlin":
         return {nm: _mm(s["x"][src], (s["w"][nm][2].double() - 8.0) * s["w"][nm][1].double().unsqueeze(1))
