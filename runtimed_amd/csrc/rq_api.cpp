@@ -289,10 +289,39 @@ static const void *aligned_x(const void *x, int xtype, int64_t m, int64_t k, hip
   return *rc ? nullptr : p;
 }
 
+// Whether a prefill call (m > 64) goes to the codes GEMM, which packs the
+// activations in a launch of its own (4-8 us) and reads them in one launch for
+// all weights, or to the tiled kernels.  Graph-timed, codes GEMM against
+// tiled, us:
+//   f32 activations, one weight: 2048 x 2048 at m = 65 / 512 18.3 / 28.2
+//     against 24.8 / 29.8 (Q4_K), 17.5 / 26.5 against 28.6 / 33.8 (Q8_0), 8192 x
+//     2048 23.9 / 67.9 against 28.7 / 73.6, 2048 x 8192 30.9 / 66.0 against
+//     62.2 / 79.5; f16 16.0 / 22.2 against 24.0 / 28.4, 51.6 against 69.8.  The
+//     pack does not pay on short rows: 896 x 896 at m = 512 19.3 against 21.7 on
+//     the K formats but 17.9 against 16.1 on Q8_0, 1152 x 384 16.7 against 11.6.
+//   Sets of weights (q/k/v, gate/up) save a launch a weight and pay throughout.
+//   bf16 activations: the tiled kernels round the weights to bf16 as well
+//     and take one matrix pass, so only sets on few tiles (m = 333: q/k/v 2048
+//     + 2 x 512 rows 29 against 50 us, m = 512: 2 x 2048 rows 35 against 32)
+//     and long rows on few tiles (896 x 4864 at m = 65 / 512 22 / 30 against 29
+//     / 32, 4096 x 4096 at m = 65 23.5 against 26.7, 2048 x 2048 16.6 against
+//     13.9, 8192 x 2048 at m = 512 54 against 33) pay.
+static bool codes_pay(const rq_weight *const *w, int count, int xtype, int64_t m) {
+  if (m <= 64) return false;
+  const int64_t k = w[0]->k;
+  int64_t tiles = 0;
+  for (int j = 0; j < count; ++j) tiles += ((w[j]->n + 63) / 64) * ((m + 63) / 64);
+  if (xtype == RQ_BF16) return count > 1 ? tiles <= 400 : k >= 4096 && tiles <= 112;
+  if (count > 1) return true;
+  const bool kfmt = w[0]->qtype == RQ_Q4_K || w[0]->qtype == RQ_Q5_K || w[0]->qtype == RQ_Q6_K;
+  return k >= (kfmt ? 896 : 1024);
+}
+
 // One weight: the fused kernels, or the generic one for shapes they do not take.
 static int linear_one(const rq_weight *w, const void *xa, int xtype, int64_t m, const Out &o, hipStream_t s,
                       WsLease &ws) {
-  int rc = launch_linear_fused(w, xa, xtype, m, o, s, ws);
+  int rc = codes_pay(&w, 1, xtype, m) ? launch_linear_codes(&w, 1, xa, xtype, m, &o, s, ws) : RQ_E_UNSUPPORTED;
+  if (rc == RQ_E_UNSUPPORTED) rc = launch_linear_fused(w, xa, xtype, m, o, s, ws);
   if (rc == RQ_E_UNSUPPORTED) rc = launch_linear_generic(w, xa, xtype, m, o, s);
   return rc;
 }
@@ -345,7 +374,9 @@ int rq_linear_multi(int count, const rq_weight *const *wts, const void *x, int x
     int j = i + 1;
     while (j < count && j - i < kMultiMax && wts[j]->qtype == wts[i]->qtype) ++j;
     for (int t = i; t < j; ++t) outs[t - i] = Out{ys[t], biases ? biases[t] : nullptr, ytype, btype};
-    rc = j - i > 1 ? launch_linear_multi(wts + i, j - i, xa, xtype, m, outs, s, ws) : RQ_E_UNSUPPORTED;
+    rc = j - i == 1                                ? RQ_E_UNSUPPORTED
+         : codes_pay(wts + i, j - i, xtype, m) ? launch_linear_codes(wts + i, j - i, xa, xtype, m, outs, s, ws)
+                                                   : launch_linear_multi(wts + i, j - i, xa, xtype, m, outs, s, ws);
     if (rc == RQ_E_UNSUPPORTED) {
       rc = RQ_OK;
       for (int t = i; t < j && !rc; ++t) rc = linear_one(wts[t], xa, xtype, m, outs[t - i], s, ws);
@@ -441,7 +472,21 @@ int rq_marlin_linear(const uint32_t *packed, const float *scales, int64_t n, int
     return set_error(RQ_E_SHAPE, "bad shape m=%lld n=%lld k=%lld", (long long)m, (long long)n, (long long)k);
   if (m == 0 || n == 0) return RQ_OK;
   if (!packed || !scales || !x || !y) return set_error(RQ_E_ARG, "null argument");
-  return launch_marlin_linear(packed, scales, n, k, x, xtype, m, y, ytype, as_stream(stream));
+  hipStream_t s = as_stream(stream);
+  // The codes GEMM (which packs x in a launch of its own) from about 2^26
+  // multiply-adds (f32 x; 2^25.3 for 16-bit x, one matrix pass): an MLP of 2048
+  // / 8192 at m = 3 / 4 / 16 58.2 / 58.8 / 60.1 us against 51.8 / 62.7 / 179.6,
+  // 4096 / 14336 at m = 2 84.5 against 88.9, 512 / 1024 at m = 32 / 64 35.9 /
+  // 40.3 against 23.6 / 43.5.
+  if (m > 1 && (double)m * (double)n * (double)k >= (xtype == RQ_F32 ? 67.0e6 : 42.0e6)) {
+    int dev = 0;
+    int rc = hip_check(hipGetDevice(&dev), "hipGetDevice");
+    if (rc) return rc;
+    WsLease ws(dev, s);
+    rc = launch_marlin_codes(packed, scales, n, k, x, xtype, m, y, ytype, s, ws);
+    if (rc != RQ_E_UNSUPPORTED) return rc;
+  }
+  return launch_marlin_linear(packed, scales, n, k, x, xtype, m, y, ytype, s);
 }
 
 static bool valid_kv_mode(int mode) { return mode == RQ_KV_F16 || mode == RQ_KV_FP8 || mode == RQ_KV_INT8; }

@@ -282,6 +282,15 @@ int launch_linear_smallm_codes(const rq_weight *const *w, int count, bool set, c
 // 64 * slices f32 / f16 activation rows as slices of 64 rows in one launch.
 int launch_linear_smallm_f32_slices(const rq_weight *wt, const void *x, int xtype, int64_t slices, const Out &o,
                                     hipStream_t s, WsLease *ws);
+// Many activation rows (prefill), 1 .. kMultiMax weights of one format and k
+// sharing x (k % 64 == 0, x 16-byte aligned): the weights' integer codes on
+// the f16 matrix cores.  RQ_E_UNSUPPORTED for other shapes, or where the
+// packed activations find no scratch.
+int launch_linear_codes(const rq_weight *const *w, int count, const void *x, int xtype, int64_t m, const Out *o,
+                        hipStream_t s, WsLease &ws);
+// The same for Marlin INT4 weights (any k and alignment of x).
+int launch_marlin_codes(const uint32_t *packed, const float *scales, int64_t n, int64_t k, const void *x, int xtype,
+                        int64_t m, void *y, int ytype, hipStream_t s, WsLease &ws);
 // Every shape and alignment: exact f32 weights decoded element by element
 // from the handle, f32 accumulation (the shapes the fused kernels do not
 // take: rows cut inside a 64-element chunk, rows longer than the GEMV
