@@ -15,10 +15,10 @@
 // A row of k inputs is P = k / piece_elems pieces.  Three layouts:
 //   segment  P <= 64: a row on an aligned segment of max(16, next_pow2(P))
 //            lanes, 64 / segment rows per wave (k_gemv_m1);
-//   team     P > 64 on n < 4096 (or more than 256 pieces): a row on a team of
-//            ceil(P / 64) waves, one piece per lane (k_gemv_team);
-//   long     P in 65..256 on n >= 4096: a row on one wave, PPL = ceil(P / 64)
-//            pieces per lane (k_gemv_long).
+//   team     P > 64: a row on a team of ceil(P / 64) waves, one piece per lane
+//            (k_gemv_team);
+//   long     P in 65..128 of a two-run format on n >= 8192: a row on one wave,
+//            two pieces per lane (k_gemv_long).
 // A lane's pieces keep the same k positions from row to row, so its
 // activations (one row, or two / four row slots for M = 2 / 3) are loaded
 // once into registers and every later row only streams weight bytes.  Rows
@@ -453,7 +453,7 @@ __device__ __forceinline__ void convert_run(int xtype, const chunk16 (&v)[4], fl
   }
 }
 
-// M = 1, long rows on fewer rows (P > 64 pieces, n < 4096): a workgroup is
+// M = 1, long rows (P > 64 pieces) the one-wave layout does not take: a workgroup is
 // one team of T = blockDim / 64 waves covering a row's pieces (piece
 // 64 tm + lane), walking the rows blockIdx.x, blockIdx.x + gridDim.x, ...
 // with D rows of weight loads in flight (static slots, unconditional loads,
@@ -672,26 +672,17 @@ int run_multi(const rq_weight *wt, const void *x, int xtype, int64_t m, const Ou
 template <class F, int PPL>
 int run_long(const rq_weight *wt, const void *x, int xtype, const Out &o, hipStream_t s) {
   // 16 waves per CU walking rows, each with two rows of weight loads in
-  // flight (measured best of 8 / 16 / 24 / 32 waves per CU).
+  // flight (measured best of 8 / 16 / 24 / 32 waves per CU), eight waves per
+  // workgroup (best of 4 / 8 / 16 on 14336 x 4096).
   const int64_t waves = wt->n < 256 * 16 ? wt->n : 256 * 16;
   const size_t xb = xlds_bytes(wt->k);
-  // Eight waves per workgroup (measured best of 4 / 8 / 16 on 14336 x 4096)
-  // for PPL <= 2; longer rows keep four (the Q6_K decode at PPL = 3 would
-  // not fit eight waves' registers).
-  if constexpr (PPL <= 2) {
-    const unsigned blocks = (unsigned)((waves + 7) / 8);
-    if (long_xr<F, PPL, 8>() > 0 && !xb) return RQ_E_UNSUPPORTED;  // k <= 64 PPL PE always fits the LDS copy
-    // Two rows in flight per wave: on Q4_K 14336 x 4096, 10.5 us against
-    // 11.9 (three rows) and 13.4 (four), whose registers leave room for one
-    // eight-wave workgroup per CU instead of two.
-    hipLaunchKernelGGL((k_gemv_long<F, PPL, 8, 2>), dim3(blocks), dim3(512), xb, s, wt->data, wt->data + wt->aux_off,
-                       x, xtype, o, wt->n, wt->k, xb != 0);
-  } else {
-    const unsigned blocks = (unsigned)((waves + 3) / 4);
-    if (long_xr<F, PPL, 4>() > 0 && !xb) return RQ_E_UNSUPPORTED;
-    hipLaunchKernelGGL((k_gemv_long<F, PPL, 4, 2>), dim3(blocks), dim3(256), xb, s, wt->data, wt->data + wt->aux_off,
-                       x, xtype, o, wt->n, wt->k, xb != 0);
-  }
+  const unsigned blocks = (unsigned)((waves + 7) / 8);
+  if (long_xr<F, PPL, 8>() > 0 && !xb) return RQ_E_UNSUPPORTED;  // k <= 64 PPL PE always fits the LDS copy
+  // Two rows in flight per wave: on Q4_K 14336 x 4096, 10.5 us against
+  // 11.9 (three rows) and 13.4 (four), whose registers leave room for one
+  // eight-wave workgroup per CU instead of two.
+  hipLaunchKernelGGL((k_gemv_long<F, PPL, 8, 2>), dim3(blocks), dim3(512), xb, s, wt->data, wt->data + wt->aux_off,
+                     x, xtype, o, wt->n, wt->k, xb != 0);
   return hipGetLastError() == hipSuccess ? RQ_OK : set_error(RQ_E_DEVICE, "gemv launch failed");
 }
 
@@ -828,16 +819,19 @@ int run_m1(const rq_weight *wt, const void *x, int xtype, const Out &o, hipStrea
       if (rc != RQ_E_UNSUPPORTED) return rc;
     }
   }
-  // Long rows on many rows: one wave per row walking the rows.
-  if (P > 64 && wt->n >= 4096) {
-    switch ((P + 63) / 64) {
-      case 2: return run_long<F, 2>(wt, x, xtype, o, s);
-      case 3: return run_long<F, 3>(wt, x, xtype, o, s);
-      case 4: return run_long<F, 4>(wt, x, xtype, o, s);
-      default: break;
-    }
+  // Rows of two pieces a lane on many rows: one wave per row walking the
+  // rows, for two-run pieces (against the team: Q4_0 / Q5_0 / Q5_K / Q8_0 14336
+  // x 4096 13.1 / 16.4 / 16.6 / 15.4 against 14.1 / 16.9 / 18.8 / 14.7 us, 8192 x
+  // 2560 7.9 / 9.7 / 9.7 / 7.9 against 9.1 / 10.6 / 11.8 / 9.0; on 4096 x 4096
+  // 8.0 / 9.5 / 10.1 / 8.9 against 6.0 / 6.9 / 7.5 / 6.7, a row a wave and no
+  // second one to overlap).
+  if constexpr (F::RUNS == 2) {
+    if (P > 64 && P <= 128 && wt->n >= 8192) return run_long<F, 2>(wt, x, xtype, o, s);
   }
-  // Other long rows: a team of waves per row.
+  // Other long rows: a team of waves per row.  A lane of the one-wave layout
+  // with more pieces holds 128 to 256 activations beside its weight slots and
+  // spills: Q6_K 4096 x 14336 69.5 us against 16.5 here, 4096 x 8192 21.9
+  // against 11.4, Q5_K / Q8_0 4096 x 8192 32.1 / 20.9 against 9.9 / 10.0.
   if (P > 64) return run_team<F, 1>(wt, x, xtype, o, s);
   return run_seg<F, 1>(wt, x, xtype, o, s);
 }
