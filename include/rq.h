@@ -48,7 +48,7 @@
  *       (crates/runtimed-model/src/ops/marlin_gemv.rs:42-202), reached through
  *       `SubstratePort::marlin_gemv` (substrate/port.rs:76) from the Marlin
  *       branch of `Weights::linear` (linear_layer.rs:53-63).
- *   rq_kv_quantize, rq_kv_dequantize
+ *   rq_kv_quantize, rq_kv_quantize_pair, rq_kv_dequantize
  *       `quantize_block_kv` / `quantize_fp8` / `quantize_int8` and
  *       `dequantize_fp8` / `dequantize_int8`
  *       (crates/runtimed-model/src/cache/paged/quantize.rs:12-123), called by
@@ -300,6 +300,11 @@ int rq_marlin_linear(const uint32_t *packed, const float *scales, int64_t n, int
  * host memory at launch time, so every shape may be captured in a graph. */
 int rq_kv_quantize(const void *t, int ttype, int64_t b, int64_t h, int64_t sd, int mode, void *q,
                    float *scales, void *stream);
+
+/* rq_kv_quantize of a K and a V chunk of one shape and type (quantize_block_kv,
+ * quantize.rs:109-135) in the same launches. */
+int rq_kv_quantize_pair(const void *k, const void *v, int ttype, int64_t b, int64_t h, int64_t sd, int mode,
+                        void *kq, void *vq, float *kscales, float *vscales, void *stream);
 
 /* dequantize_fp8 / dequantize_int8 (quantize.rs:48-57, 98-107): out =
  * decode(q) * scales[h] (f32 product) as otype (F32, F16 or BF16); RQ_KV_F16

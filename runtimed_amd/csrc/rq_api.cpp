@@ -491,26 +491,44 @@ int rq_marlin_linear(const uint32_t *packed, const float *scales, int64_t n, int
 
 static bool valid_kv_mode(int mode) { return mode == RQ_KV_F16 || mode == RQ_KV_FP8 || mode == RQ_KV_INT8; }
 
-int rq_kv_quantize(const void *t, int ttype, int64_t b, int64_t h, int64_t sd, int mode, void *q, float *scales,
-                   void *stream) {
+static int kv_quantize(int count, const void *const *t, int ttype, int64_t b, int64_t h, int64_t sd, int mode,
+                       void *const *q, float *const *scales, void *stream) {
   g_last_error.clear();
   if (!valid_ftype(ttype)) return set_error(RQ_E_ARG, "input type %d not supported", ttype);
   if (!valid_kv_mode(mode)) return set_error(RQ_E_ARG, "bad kv mode %d", mode);
   if (b < 0 || h < 0 || sd < 0)
     return set_error(RQ_E_SHAPE, "bad shape [%lld, %lld, %lld]", (long long)b, (long long)h, (long long)sd);
   if (h == 0) return RQ_OK;
-  if (!scales) return set_error(RQ_E_ARG, "null scales");
+  for (int i = 0; i < count; ++i)
+    if (!scales[i]) return set_error(RQ_E_ARG, "null scales");
   if (b == 0 || sd == 0) {
     // No elements: every head's maximum is 0, so its scale is the floor,
     // written by a kernel (nothing read from host memory at replay time).
-    return launch_kv_fill_scales(scales, h, mode == RQ_KV_F16 ? 1.0f : 1e-8f, as_stream(stream));
+    int rc = RQ_OK;
+    for (int i = 0; i < count && !rc; ++i)
+      rc = launch_kv_fill_scales(scales[i], h, mode == RQ_KV_F16 ? 1.0f : 1e-8f, as_stream(stream));
+    return rc;
   }
-  if (!t || !q) return set_error(RQ_E_ARG, "null argument");
+  for (int i = 0; i < count; ++i)
+    if (!t[i] || !q[i]) return set_error(RQ_E_ARG, "null argument");
   int dev = 0;
   const int rc = hip_check(hipGetDevice(&dev), "hipGetDevice");
   if (rc) return rc;
   WsLease ws(dev, as_stream(stream));
-  return launch_kv_quantize(t, ttype, b, h, sd, mode, q, scales, as_stream(stream), ws);
+  return launch_kv_quantize(count, t, ttype, b, h, sd, mode, q, scales, as_stream(stream), ws);
+}
+
+int rq_kv_quantize(const void *t, int ttype, int64_t b, int64_t h, int64_t sd, int mode, void *q, float *scales,
+                   void *stream) {
+  return kv_quantize(1, &t, ttype, b, h, sd, mode, &q, &scales, stream);
+}
+
+int rq_kv_quantize_pair(const void *k, const void *v, int ttype, int64_t b, int64_t h, int64_t sd, int mode, void *kq,
+                        void *vq, float *kscales, float *vscales, void *stream) {
+  const void *const t[2] = {k, v};
+  void *const q[2] = {kq, vq};
+  float *const scales[2] = {kscales, vscales};
+  return kv_quantize(2, t, ttype, b, h, sd, mode, q, scales, stream);
 }
 
 int rq_kv_dequantize(const void *q, int mode, const float *scales, int64_t b, int64_t h, int64_t sd, void *out,

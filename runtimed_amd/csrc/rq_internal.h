@@ -312,8 +312,9 @@ int launch_marlin_dequant(const uint32_t *packed, const float *s, int64_t n, int
 int launch_marlin_linear(const uint32_t *packed, const float *s, int64_t n, int64_t k, const void *x, int xtype,
                          int64_t m, void *y, int ytype, hipStream_t st);
 // Paged-KV block quantizer (arguments validated by the caller).
-int launch_kv_quantize(const void *t, int ttype, int64_t b, int64_t h, int64_t sd, int mode, void *q,
-                       float *scales, hipStream_t s, WsLease &ws);
+// One tensor or two of equal shape and type (count 1 or 2) in the same launches.
+int launch_kv_quantize(int count, const void *const *t, int ttype, int64_t b, int64_t h, int64_t sd, int mode,
+                       void *const *q, float *const *scales, hipStream_t s, WsLease &ws);
 int launch_kv_dequantize(const void *q, int mode, const float *scales, int64_t b, int64_t h, int64_t sd, void *out,
                          int otype, hipStream_t s);
 // scales[0 .. h) = v on the stream (a kernel: safe under graph capture).

@@ -81,6 +81,7 @@ def lib() -> ctypes.CDLL:
         L.rq_marlin_dequant.argtypes = [vp, vp, i64, i64, vp, vp]
         L.rq_marlin_linear.argtypes = [vp, vp, i64, i64, vp, i32, i64, vp, i32, vp]
         L.rq_kv_quantize.argtypes = [vp, i32, i64, i64, i64, i32, vp, vp, vp]
+        L.rq_kv_quantize_pair.argtypes = [vp, vp, i32, i64, i64, i64, i32, vp, vp, vp, vp, vp]
         L.rq_kv_dequantize.argtypes = [vp, i32, vp, i64, i64, i64, vp, i32, vp]
         for f in ("rq_weight_create", "rq_weight_info", "rq_dequant_f32", "rq_dequant_tensor",
                   "rq_linear", "rq_linear_bias", "rq_linear_multi", "rq_bias_add", "rq_fp8_quantize",
@@ -343,15 +344,30 @@ def _kv_input(t: torch.Tensor) -> torch.Tensor:
     return t if t.dtype in (torch.float32, torch.float16, torch.bfloat16) else t.to(torch.float32)
 
 
+_KV_CODES = {KV_FP8: torch.float8_e4m3fn, KV_INT8: torch.uint8, KV_F16: torch.float16}
+
+
 def _kv_quantize(t: torch.Tensor, mode: int):
     b, h, sd = _kv_dims(t)
     src = _kv_input(t)
-    qdt = {KV_FP8: torch.float8_e4m3fn, KV_INT8: torch.uint8, KV_F16: torch.float16}[mode]
-    q = torch.empty(t.shape, dtype=qdt, device=t.device)
+    q = torch.empty(t.shape, dtype=_KV_CODES[mode], device=t.device)
     s = torch.empty(h, dtype=torch.float32, device=t.device)
     check(lib().rq_kv_quantize(_ptr(src), ftype(src.dtype), b, h, sd, mode, _ptr(q), _ptr(s),
                                _stream(t.device)))
     return q, s.reshape(1, h, 1, 1)
+
+
+def _kv_quantize_pair(k: torch.Tensor, v: torch.Tensor, mode: int):
+    """_kv_quantize of both, in the same launches where shape, type and device agree."""
+    if k.shape != v.shape or k.dtype != v.dtype or k.device != v.device:
+        return (*_kv_quantize(k, mode), *_kv_quantize(v, mode))
+    b, h, sd = _kv_dims(k)
+    ks, vs = _kv_input(k), _kv_input(v)
+    kq, vq = (torch.empty(k.shape, dtype=_KV_CODES[mode], device=k.device) for _ in range(2))
+    sk, sv = (torch.empty(h, dtype=torch.float32, device=k.device) for _ in range(2))
+    check(lib().rq_kv_quantize_pair(_ptr(ks), _ptr(vs), ftype(ks.dtype), b, h, sd, mode, _ptr(kq), _ptr(vq), _ptr(sk),
+                                    _ptr(sv), _stream(k.device)))
+    return kq, sk.reshape(1, h, 1, 1), vq, sv.reshape(1, h, 1, 1)
 
 
 def quantize_fp8(t: torch.Tensor):
@@ -389,14 +405,12 @@ def quantize_block_kv(token_offset: int, k: torch.Tensor, v: torch.Tensor, reque
     """quantize_block_kv (quantize.rs:109-135): the first SINK_TOKENS_COUNT
     tokens, and Fp16 caches, stay f16 with scale 1."""
     if token_offset < SINK_TOKENS_COUNT or requested_precision == KV_F16:
-        kf, _ = _kv_quantize(k, KV_F16)
-        vf, _ = _kv_quantize(v, KV_F16)
+        kf, _, vf, _ = _kv_quantize_pair(k, v, KV_F16)
         one_k = torch.ones(1, dtype=torch.float32, device=k.device)
         one_v = torch.ones(1, dtype=torch.float32, device=v.device)
         return kf, vf, one_k, one_v, KV_F16
     mode = KV_INT8 if requested_precision == KV_INT8 else KV_FP8
-    kq, ks = _kv_quantize(k, mode)
-    vq, vs = _kv_quantize(v, mode)
+    kq, ks, vq, vs = _kv_quantize_pair(k, v, mode)
     return kq, vq, ks, vs, mode
 
 
