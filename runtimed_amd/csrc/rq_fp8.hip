@@ -61,8 +61,8 @@ __global__ __launch_bounds__(256) void k_fp8_quant_rows(const void *__restrict__
   if (tid == 0) xs[row] = amax / 448.0f;
 }
 
-// The same per-token encode with one wave per activation row (four rows a
-// workgroup): the row's maximum from 16-byte loads and a wave reduction,
+// The same per-token encode with WPR waves per activation row (one, four rows
+// a workgroup, or four): the row's maximum from 16-byte loads and a wave reduction,
 // then the codes from a second pass over the row (an L2 hit, or the
 // registers when the row is at most one batch), 4 (f32) or 8 (f16 / bf16)
 // codes per store.  Same codes and scales as k_fp8_quant_rows (the maximum
@@ -70,13 +70,14 @@ __global__ __launch_bounds__(256) void k_fp8_quant_rows(const void *__restrict__
 // activation type and the mode are template parameters: as run-time values
 // the compiler turned each per-element choice into a branch.  One workgroup
 // per row with scalar 2-byte loads took 21 us on 2048 x 4096 bf16.
-template <int XT, bool SCALED>
+template <int XT, bool SCALED, int WPR>
 __global__ __launch_bounds__(256) void k_fp8_quant_waves(const void *__restrict__ x, int64_t m, int64_t k,
                                                         uint8_t *__restrict__ xq, float *__restrict__ xs) {
   constexpr bool F32X = XT == RQ_F32;
   constexpr int ES = F32X ? 4 : 8;  // elements per 16-byte chunk
-  const int lane = threadIdx.x & 63;
-  const int64_t row = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+  constexpr int T = 64 * WPR;  // threads a row
+  const int lane = (int)threadIdx.x & (T - 1);
+  const int64_t row = (int64_t)blockIdx.x * (4 / WPR) + threadIdx.x / T;
   if (row >= m) return;
   const int64_t nch = k / ES;
   const uint4 *src = reinterpret_cast<const uint4 *>(static_cast<const uint8_t *>(x) + row * k * (F32X ? 4 : 2));
@@ -97,26 +98,26 @@ __global__ __launch_bounds__(256) void k_fp8_quant_waves(const void *__restrict_
   };
   // Batches of U chunks a lane, their loads issued together; a row of at
   // most one batch stays in registers between the two passes.
-  constexpr int U = 8;
+  constexpr int U = WPR == 1 ? 1 : 4;
   uint4 buf[U];
   auto load_batch = [&](int64_t c0) {
 #pragma unroll
     for (int u = 0; u < U; ++u) {
-      const int64_t c = c0 + 64 * u;
+      const int64_t c = c0 + T * u;
       buf[u] = src[c < nch ? c : nch - 1];
     }
   };
-  const bool resident = SCALED && nch <= 64 * U;
+  const bool resident = SCALED && nch <= T * U;
   float amax = 0.0f;
   bool nan = false;
   if constexpr (SCALED) {
-    for (int64_t c0 = lane; c0 < nch; c0 += 64 * U) {
+    for (int64_t c0 = lane; c0 < nch; c0 += T * U) {
       load_batch(c0);
 #pragma unroll
       for (int u = 0; u < U; ++u) {
         float f[ES];
         unpack(buf[u], f);
-        const bool live = c0 + 64 * u < nch;
+        const bool live = c0 + T * u < nch;
 #pragma unroll
         for (int i = 0; i < ES; ++i) {
           amax = fmaxf(amax, live ? fabsf(f[i]) : 0.0f);
@@ -126,6 +127,15 @@ __global__ __launch_bounds__(256) void k_fp8_quant_waves(const void *__restrict_
     }
 #pragma unroll
     for (int off = 32; off > 0; off >>= 1) amax = fmaxf(amax, __shfl_xor(amax, off));
+    nan = __any(nan);
+    if constexpr (WPR > 1) {
+      __shared__ float red[WPR];
+      __shared__ int bad[WPR];
+      if ((lane & 63) == 0) red[lane >> 6] = amax, bad[lane >> 6] = nan;
+      __syncthreads();
+#pragma unroll
+      for (int i = 0; i < WPR; ++i) amax = fmaxf(amax, red[i]), nan |= bad[i] != 0;
+    }
   }
   // A row without NaN is encoded by the hardware conversion: for |v| <= 448
   // v_cvt_pk_fp8_f32 gives enc_e4m3_rne's code for every f32 input (compared
@@ -133,17 +143,17 @@ __global__ __launch_bounds__(256) void k_fp8_quant_waves(const void *__restrict_
   // product can exceed 448 by an ulp).  Rows with a NaN or an infinity (whose
   // product with inv = 0 is NaN) keep the software encoder, whose NaN code
   // differs.
-  const bool hw = SCALED && !__any(nan) && amax != 0.0f && amax <= 3.4028235e38f;  // no NaN, no infinity
+  const bool hw = SCALED && !nan && amax != 0.0f && amax <= 3.4028235e38f;  // no NaN, no infinity
   // amax == 0: every code 0 (inv = 0 would turn NaN or infinite inputs into
   // NaN codes instead).
   const float inv = 448.0f / amax;
   const uint32_t keep = amax == 0.0f ? 0u : 0xFFu;
   uint8_t *dst = xq + row * k;
-  for (int64_t c0 = lane; c0 < nch; c0 += 64 * U) {
+  for (int64_t c0 = lane; c0 < nch; c0 += T * U) {
     if (!resident) load_batch(c0);
 #pragma unroll
     for (int u = 0; u < U; ++u) {
-      const int64_t c = c0 + 64 * u;
+      const int64_t c = c0 + T * u;
       float f[ES];
       unpack(buf[u], f);
       uint32_t word[ES / 4];
@@ -176,7 +186,8 @@ __global__ __launch_bounds__(256) void k_fp8_quant_waves(const void *__restrict_
   if (lane == 0) xs[row] = !SCALED ? 1.0f : amax == 0.0f ? 0.0f : amax / 448.0f;
 }
 
-// Scalar fallback for shapes the tiled kernel does not take (k % 128 != 0).
+// Scalar fallback for shapes the matrix-core kernels do not take (k % 16 != 0
+// or misaligned operands).
 __global__ __launch_bounds__(256) void k_fp8_gemm_scalar(const uint8_t *__restrict__ xq,
                                                         const float *__restrict__ xs, int64_t m,
                                                         const uint8_t *__restrict__ w,
@@ -293,6 +304,134 @@ __global__ __launch_bounds__(256) void k_fp8_gemm_mfma(const uint8_t *__restrict
                          sw[J], nob, xs, ws, lane, vec);
     });
   });
+}
+
+// ---- few tiles: 16 MT rows x 32 columns a workgroup, K split over its waves ----
+//
+// Decode and verify rows (and more rows on narrow weights) leave the 128 x 128
+// tiles on a fraction of the CUs, each walking the whole of K behind one
+// barrier a step.  Here a workgroup owns 16 MT rows of x and 32 rows of w; its
+// waves share K in steps of 128 inputs, each with its operands straight from
+// global memory (no LDS, no barrier until the waves' sums meet): a lane loads
+// two 16-byte pieces a row and step, four lanes 64 consecutive bytes of a row.
+// One step of loads a wave is in flight: the wave then fits eight to a SIMD (48
+// registers at MT = 1), which hides more than two, three or four steps in fewer
+// waves did (5 x 14336 x 4096: 16.9 us against 17.7 / 24.5 / 18.7).  Plain loads:
+// with non-temporal ones each half of a 128-byte line went to memory by itself
+// (17.1 us against 13.1).  The order of the inputs inside a step
+// is the same for both operands, so it need not be the natural one.  The
+// codes are widened to f16, exactly, and the products summed on the f16 matrix
+// cores: for these sizes as fast as the fp8 ones within 10 % and without their
+// truncated sums (error against 64 bits 6e-8 instead of 1.4e-5).  Bound: the
+// weight bytes (HBM) for few rows; 5 x 14336 x 4096 30.6 -> 13.1 us (4.5 TB/s),
+// 5 x 4096 x 4096 30.1 -> 7.7, 512 x 2048 x 4096 29.9 -> 26.9, 100 x 2000 x 2048
+// 20.9 -> 10.1 against the 128 x 128 tiles, 100 x 3000 x 2016 2479 -> 8.2 against
+// one thread an output.  A row of x past m or of w past n
+// re-reads the last one; its results are not stored.  TAIL: k % 128 != 0 (k %
+// 16 == 0).
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
+typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
+
+template <int MT, bool TAIL>
+__global__ __launch_bounds__(512) void k_fp8_skinny(const uint8_t *__restrict__ a, const float *__restrict__ xs,
+                                                    int64_t m, const uint8_t *__restrict__ b,
+                                                    const float *__restrict__ ws, int64_t n, int64_t k,
+                                                    void *__restrict__ y, int ytype, int tm) {
+    extern __shared__ __attribute__((aligned(16))) float red[];  // [wave][2 MT tiles][4][64]
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int W = (int)(blockDim.x >> 6);
+  // XCD x (workgroups x, x + 8, ..) takes a run of consecutive tiles, rows of
+  // x fastest, so that tiles sharing weights share an L2.
+  const int T = (int)gridDim.x, xcd = (int)blockIdx.x & 7, qt = T >> 3, rt = T & 7;
+  const int unit = xcd * qt + (xcd < rt ? xcd : rt) + ((int)blockIdx.x >> 3);
+  const int nt = unit / tm, mt = unit - nt * tm;
+  const int64_t m0 = 16 * MT * (int64_t)mt, n0 = 32 * (int64_t)nt;
+  const int steps = (int)((k + 127) / 128);
+  const int s0 = (int)((int64_t)steps * wave / W), s1 = (int)((int64_t)steps * (wave + 1) / W);
+  const int r = lane & 15, g = lane >> 4;
+
+  // Uniform tile bases, 32-bit lane offsets (32 or 64 rows of k <= 2^24 bytes).
+  const uint8_t *const ta = a + m0 * k, *const tb = b + n0 * k;
+  uint32_t oa[MT], ob[2];
+#pragma unroll
+  for (int i = 0; i < MT; ++i) oa[i] = (uint32_t)(m0 + 16 * i + r < m ? 16 * i + r : (int)(m - 1 - m0)) * (uint32_t)k;
+#pragma unroll
+  for (int j = 0; j < 2; ++j) ob[j] = (uint32_t)(n0 + 16 * j + r < n ? 16 * j + r : (int)(n - 1 - n0)) * (uint32_t)k;
+  u32x4 fa[MT][2], fb[2][2];
+  const int last = s1 > s0 ? s1 - 1 : 0;
+  auto fill = [&](int s) __attribute__((always_inline)) {
+    const int base = 128 * (s < last ? s : last);
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const int o = base + 16 * g + 64 * h;
+      const uint32_t oc = !TAIL || o < (int)k ? o : 0;
+#pragma unroll
+      for (int j = 0; j < 2; ++j) fb[j][h] = *reinterpret_cast<const u32x4 *>(tb + (ob[j] + oc));
+#pragma unroll
+      for (int i = 0; i < MT; ++i) fa[i][h] = *reinterpret_cast<const u32x4 *>(ta + (oa[i] + oc));
+    }
+  };
+  // Eight codes of a piece (half h) in f16, exactly.
+  auto wide = [](const u32x4 &x, int h) __attribute__((always_inline)) {
+    const uint32_t w0 = h ? x.z : x.x, w1 = h ? x.w : x.y;
+    const f16x2 v0 = __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(w0, 1.0f, false);
+    const f16x2 v1 = __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(w0, 1.0f, true);
+    const f16x2 v2 = __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(w1, 1.0f, false);
+    const f16x2 v3 = __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(w1, 1.0f, true);
+    return (f16x8){v0[0], v0[1], v1[0], v1[1], v2[0], v2[1], v3[0], v3[1]};
+  };
+  f32x4 acc[MT][2];
+#pragma unroll
+  for (int i = 0; i < MT; ++i)
+#pragma unroll
+    for (int j = 0; j < 2; ++j) acc[i][j] = (f32x4){0, 0, 0, 0};
+  auto emit = [&](int s) __attribute__((always_inline)) {
+    // Pieces past k hold the row's first piece: zeros in x's (w's codes are
+    // finite there, or the row's sum is a NaN in any case).
+    if (TAIL && s == steps - 1) {
+#pragma unroll
+      for (int h = 0; h < 2; ++h)
+#pragma unroll
+        for (int i = 0; i < MT; ++i)
+          if (128 * s + 16 * g + 64 * h >= (int)k) fa[i][h] = (u32x4){0, 0, 0, 0};
+    }
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+#pragma unroll
+      for (int p = 0; p < 4; ++p) {
+        const f16x8 ob8 = wide(fb[j][p >> 1], p & 1);
+#pragma unroll
+        for (int i = 0; i < MT; ++i)
+          acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(wide(fa[i][p >> 1], p & 1), ob8, acc[i][j], 0, 0, 0);
+      }
+  };
+  fill(s0);
+  for (int s = s0; s < s1; ++s) {
+    emit(s);
+    fill(s + 1);
+  }
+
+  // The waves' tiles summed in wave order.  Slot q of the tile: MFMA tile
+  // q / 4 (row tile q / 8, column tile (q / 4) % 2), element q % 4: rows 16 i
+  // + 4 (lane / 16) + q % 4, column 16 j + lane % 16.
+  constexpr int Q = 8 * MT;
+#pragma unroll
+  for (int i = 0; i < MT; ++i)
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) red[(wave * Q + (2 * i + j) * 4 + e) * 64 + lane] = acc[i][j][e];
+  __syncthreads();
+  for (int q = wave; q < Q; q += W) {
+    const int64_t row = m0 + 16 * (q >> 3) + 4 * (lane >> 4) + (q & 3);
+    const int64_t col = n0 + 16 * ((q >> 2) & 1) + (lane & 15);
+    if (row < m && col < n) {
+      float v = red[q * 64 + lane];
+      for (int w = 1; w < W; ++w) v += red[(w * Q + q) * 64 + lane];
+      store_out(y, ytype, row * n + col, v * ((xs ? xs[row] : 1.0f) * (ws ? ws[col] : 1.0f)));
+    }
+  }
 }
 
 // ---- pipelined 256 x 256 kernel ------------------------------------------
@@ -602,12 +741,23 @@ __global__ __launch_bounds__(512) void k_fp8_gemm_pipe8(const uint8_t *__restric
   });
 }
 
-template <int BM, int BN, int WM, int WN, int BK>
 void launch_tiled(const uint8_t *xq, const float *xs, int64_t m, const uint8_t *w, const float *ws,
                   int64_t n, int64_t k, void *y, int ytype, hipStream_t s) {
-  const dim3 grid((unsigned)((n + BN - 1) / BN), (unsigned)((m + BM - 1) / BM));
-  hipLaunchKernelGGL((k_fp8_gemm_mfma<BM, BN, WM, WN, BK>), grid, dim3(256), 0, s, xq, xs, m, w, ws, n, k, y,
-                     ytype);
+  const dim3 grid((unsigned)((n + 127) / 128), (unsigned)((m + 127) / 128));
+  hipLaunchKernelGGL((k_fp8_gemm_mfma<128, 128, 2, 2, 128>), grid, dim3(256), 0, s, xq, xs, m, w, ws, n, k, y, ytype);
+}
+
+template <int MT>
+void launch_skinny(const uint8_t *xq, const float *xs, int64_t m, const uint8_t *w, const float *ws, int64_t n,
+                   int64_t k, void *y, int ytype, hipStream_t s) {
+  const int64_t tm = (m + 16 * MT - 1) / (16 * MT), wgs = tm * ((n + 31) / 32), steps = (k + 127) / 128;
+  const int waves = (int)(steps < 8 ? steps : 8);
+  const size_t lds = (size_t)waves * MT * 2048;  // at most 64 KB
+#define RQ_SK(TAIL)                                                                                              \
+  hipLaunchKernelGGL((k_fp8_skinny<MT, TAIL>), dim3((unsigned)wgs), dim3(64 * waves), lds, s, xq, xs, m, w, ws, n, k, y, \
+                     ytype, (int)tm)
+  if (k % 128 == 0) RQ_SK(false); else RQ_SK(true);
+#undef RQ_SK
 }
 
 }  // namespace
@@ -620,15 +770,21 @@ int launch_fp8_quantize(const void *x, int xtype, int64_t m, int64_t k, int mode
   const bool vec = reinterpret_cast<uintptr_t>(x) % 16 == 0 && k % es == 0 && (k * (f32x ? 4 : 2)) % 16 == 0 &&
                    reinterpret_cast<uintptr_t>(xq) % es == 0;
   if (vec) {
-    const dim3 grid((unsigned)((m + 3) / 4));
     const bool sc = mode != RQ_FP8_UNSCALED;
-#define RQ_QW(XT, SC) hipLaunchKernelGGL((k_fp8_quant_waves<XT, SC>), grid, dim3(256), 0, s, x, m, k, xq, xs)
+    // Four waves a row unless one wave holds it in one chunk a lane (k = 4096,
+    // f32: m = 5 4.3 -> 2.7 us, 512 4.8 -> 3.3, 2048 7.8 -> 6.9 against one wave
+    // a row).
+    const bool wide = k / es > 64;
+    const dim3 grid((unsigned)(wide ? m : (m + 3) / 4));
+#define RQ_QW(XT, SC)                                                                                                \
+  if (wide) hipLaunchKernelGGL((k_fp8_quant_waves<XT, SC, 4>), grid, dim3(256), 0, s, x, m, k, xq, xs);              \
+  else hipLaunchKernelGGL((k_fp8_quant_waves<XT, SC, 1>), grid, dim3(256), 0, s, x, m, k, xq, xs)
     if (xtype == RQ_F32) {
-      if (sc) RQ_QW(RQ_F32, true); else RQ_QW(RQ_F32, false);
+      if (sc) { RQ_QW(RQ_F32, true); } else { RQ_QW(RQ_F32, false); }
     } else if (xtype == RQ_BF16) {
-      if (sc) RQ_QW(RQ_BF16, true); else RQ_QW(RQ_BF16, false);
+      if (sc) { RQ_QW(RQ_BF16, true); } else { RQ_QW(RQ_BF16, false); }
     } else {
-      if (sc) RQ_QW(RQ_F16, true); else RQ_QW(RQ_F16, false);
+      if (sc) { RQ_QW(RQ_F16, true); } else { RQ_QW(RQ_F16, false); }
     }
 #undef RQ_QW
   } else {
@@ -642,7 +798,14 @@ int launch_fp8_gemm(const uint8_t *xq, const float *xs, int64_t m, const uint8_t
   if (m == 0 || n == 0) return RQ_OK;
   const bool aligned = (reinterpret_cast<uintptr_t>(xq) % 16 == 0) &&
                        (reinterpret_cast<uintptr_t>(w) % 16 == 0);
-  if (k % 128 == 0 && aligned) {
+  // 16 MT x 32 tiles with K split over a workgroup's waves where the 128 x 128
+  // tiles would leave CUs idle: up to 512 workgroups of 64 x 32 (at k = 4096 512
+  // x 2048 26.9 against 29.9 us and 64 x 14336 31.2 against 30.8; 128 x 14336
+  // 48.4 against 32.6), all of at most 32 rows (24 x 14336 17.8 against 33.4),
+  // and every k that is not a multiple of 128.
+  const int64_t sk_wgs = ((m + 63) / 64) * ((n + 31) / 32);
+  const bool sk_ok = k % 16 == 0 && k <= (1 << 24) && sk_wgs <= 0x3FFFFFFF;
+  if (aligned && k % 128 == 0 && !(sk_ok && (m <= 32 || sk_wgs <= 512))) {
     // 256 x 256 tiles when there are enough of them to cover the CUs (eight
     // waves of 128 x 64 for whole groups of four K-steps, else four of
     // 128 x 128), else 128 x 128.
@@ -654,8 +817,12 @@ int launch_fp8_gemm(const uint8_t *xq, const float *xs, int64_t m, const uint8_t
       else
         hipLaunchKernelGGL(k_fp8_gemm_pipe, grid, dim3(256), 0, s, xq, xs, m, w, ws, n, k, y, ytype);
     } else {
-      launch_tiled<128, 128, 2, 2, 128>(xq, xs, m, w, ws, n, k, y, ytype, s);
+      launch_tiled(xq, xs, m, w, ws, n, k, y, ytype, s);
     }
+  } else if (aligned && sk_ok) {
+    if (m <= 16) launch_skinny<1>(xq, xs, m, w, ws, n, k, y, ytype, s);
+    else if (m <= 32) launch_skinny<2>(xq, xs, m, w, ws, n, k, y, ytype, s);
+    else launch_skinny<4>(xq, xs, m, w, ws, n, k, y, ytype, s);
   } else {
     const int64_t total = m * n;
     hipLaunchKernelGGL(k_fp8_gemm_scalar, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, s, xq,
