@@ -1,7 +1,8 @@
-"""Build librq.so (the HIP kernels and the C ABI of include/rq.h) for gfx950.
+"""Build librq.so (the HIP kernels and the C ABI of include/rq.h) for gfx950
+and _rqc.so, the Python extension on it.
 
 Run as ``python -m runtimed_amd.build`` or through ``__graft_entry__.build()``.
-Objects go to runtimed_amd/_build/, the library to runtimed_amd/librq.so.
+Objects go to runtimed_amd/_build/, the libraries to runtimed_amd/.
 """
 from __future__ import annotations
 
@@ -9,6 +10,7 @@ import concurrent.futures
 import os
 import subprocess
 import sys
+import sysconfig
 import time
 from pathlib import Path
 
@@ -16,7 +18,10 @@ PKG = Path(__file__).resolve().parent
 CSRC = PKG / "csrc"
 OUT = PKG / "_build"
 LIB = PKG / "librq.so"
+BIND_SRC = CSRC / "rq_bind.cpp"
+BIND = PKG / "_rqc.so"
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
+ROCM = Path(os.environ.get("ROCM_PATH", "/opt/rocm"))
 ARCH = "gfx950"
 
 SOURCES = ["csrc/rq_api.cpp", "csrc/rq_dequant.hip", "csrc/rq_gemv.hip", "csrc/rq_gemv_mx.hip", "csrc/rq_fp8.hip",
@@ -46,6 +51,28 @@ def _compile(src: str) -> Path:
     return obj
 
 
+def _build_bind() -> None:
+    """The Python extension of csrc/rq_bind.cpp, against torch's and Python's headers; finds librq.so beside it."""
+    import torch
+
+    t = Path(torch.__file__).resolve().parent
+    tmp = BIND.with_suffix(".so.tmp")
+    cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
+           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", f"-isystem{t}/include",
+           f"-isystem{t}/include/torch/csrc/api/include", f"-isystem{ROCM}/include",
+           f"-isystem{sysconfig.get_paths()['include']}", str(BIND_SRC), "-o", str(tmp), f"-L{t}/lib", "-lc10",
+           "-lc10_hip", "-ltorch_cpu", "-ltorch_python", f"-L{PKG}", "-lrq", "-Wl,-rpath,$ORIGIN"]
+    res = subprocess.run(cmd, capture_output=True, text=True)
+    if res.returncode != 0:
+        raise RuntimeError(f"binding build failed:\n{res.stderr}")
+    os.replace(tmp, BIND)
+
+
+def _bind_stale() -> bool:
+    deps = [BIND_SRC, ROOT / "include" / "rq.h"]
+    return not BIND.exists() or any(d.stat().st_mtime > BIND.stat().st_mtime for d in deps)
+
+
 def _stale(src: str) -> bool:
     """An object older than its source or than any header it may include."""
     obj = OUT / (Path(src).stem + ".o")
@@ -70,6 +97,8 @@ def build(verbose: bool = False, incremental: bool = False) -> Path:
     if res.returncode != 0:
         raise RuntimeError(f"link failed:\n{res.stderr}")
     os.replace(tmp, LIB)
+    if not incremental or _bind_stale():
+        _build_bind()
     if verbose:
         print(f"built {LIB}")
     return LIB

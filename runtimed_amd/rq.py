@@ -8,6 +8,7 @@ fallback path.
 from __future__ import annotations
 
 import ctypes
+import importlib
 from pathlib import Path
 from typing import Optional
 
@@ -91,6 +92,29 @@ def lib() -> ctypes.CDLL:
     return _lib
 
 
+_rqc = None
+
+
+def _native():
+    """The extension that runs the plain form of a call without ctypes (csrc/rq_bind.cpp): each of its
+    functions returns the outputs, a negative rq_status, or None where the call is not of that form."""
+    global _rqc
+    if _rqc is None:
+        lib()
+        try:
+            _rqc = importlib.import_module(__package__ + "._rqc")
+        except ImportError as e:
+            raise RuntimeError(f"the binding is not built; run `python -m runtimed_amd.build` ({e})") from e
+    return _rqc
+
+
+def _done(r):
+    """Outputs of a native call; raises for a status."""
+    if r.__class__ is int:
+        check(r)
+    return r
+
+
 def check(rc: int) -> None:
     if rc != 0:
         raise RqError(rc, lib().rq_last_error().decode())
@@ -122,13 +146,13 @@ class QWeight:
         h = ctypes.c_void_p()
         check(lib().rq_weight_create(qtype, buf.ctypes.data_as(ctypes.c_void_p), buf.nbytes, n, k,
                                      device, ctypes.byref(h)))
-        self._h = h
+        self._h, self._hv = h, h.value
         self.qtype, self.n, self.k, self.device = qtype, n, k, torch.device("cuda", device)
 
     def close(self) -> None:
         if getattr(self, "_h", None) and self._h.value:
             lib().rq_weight_destroy(self._h)
-            self._h = ctypes.c_void_p()
+            self._h, self._hv = ctypes.c_void_p(), 0
 
     def __del__(self):
         try:
@@ -153,16 +177,17 @@ class QWeight:
     def embedding(self, ids) -> torch.Tensor:
         """Rows `ids` decoded exactly, f32 [len(ids), k] (embed_layer.rs:16-84)."""
         ids = np.ascontiguousarray(np.asarray(ids, dtype=np.uint32).reshape(-1))
-        out = torch.empty((ids.size, self.k), dtype=torch.float32, device=self.device)
-        check(lib().rq_embedding(self._h, ids.ctypes.data_as(ctypes.c_void_p), ids.size, _ptr(out),
-                                 _stream(self.device)))
-        return out
+        return _done((_rqc or _native()).embedding(self._hv, self.k, self.device.index, ids))
 
     def forward(self, x: torch.Tensor, out_dtype: Optional[torch.dtype] = None,
                 out: Optional[torch.Tensor] = None, bias: Optional[torch.Tensor] = None) -> torch.Tensor:
         """y = x W^T (+ bias) over the last dimension of x (linear_layer.rs:45-52,
         107-118).  A last dimension other than k raises Shape from the library
         (linear_layer.rs:88-96)."""
+        if out is None:
+            r = (_rqc or _native()).linear(self, x, out_dtype, bias)
+            if r is not None:
+                return _done(r)
         k = x.shape[-1] if x.dim() else 0
         if not x.is_contiguous():
             x = x.contiguous()
@@ -181,6 +206,9 @@ class QWeight:
 def linear_multi(weights, x: torch.Tensor, biases=None, out_dtype: Optional[torch.dtype] = None):
     """Several linears on one input (q/k/v, gate/up: qwen2.rs:99-125) through
     rq_linear_multi; returns the outputs in order."""
+    r = (_rqc or _native()).linear_multi(weights, x, biases, out_dtype)
+    if r is not None:
+        return _done(r)
     x = x.contiguous()
     outs = [torch.empty((*x.shape[:-1], w.n), dtype=out_dtype or x.dtype, device=x.device) for w in weights]
     if outs:
@@ -235,6 +263,10 @@ def fp8_gemm(x: torch.Tensor, w: torch.Tensor, w_scale: Optional[torch.Tensor],
              mode: int = FP8_PER_TOKEN, out_dtype: torch.dtype = torch.bfloat16,
              out: Optional[torch.Tensor] = None) -> torch.Tensor:
     """y = x (w * w_scale)^T with e4m3 w codes [n, k] (fp8_gemm.rs:77-191)."""
+    if out is None:
+        r = (_rqc or _native()).fp8_gemm(x, w, w_scale, mode, out_dtype)
+        if r is not None:
+            return _done(r)
     n, k = w.shape
     if x.shape[-1] != k:
         raise RqError(-4, f"expected last dim {k}, got {list(x.shape)}")
@@ -315,6 +347,9 @@ def repack_marlin_tiles(weight: torch.Tensor, scales: torch.Tensor) -> MarlinWei
 def marlin_gemv(x: torch.Tensor, w: MarlinWeight) -> torch.Tensor:
     """x @ (w * scale)^T over the last dimension of x, result in x's dtype
     (marlin_gemv.rs:119-202)."""
+    r = (_rqc or _native()).marlin(x, w.packed, w.scales, w.in_dim, w.out_dim)
+    if r is not None:
+        return _done(r)
     in_dim = x.shape[-1] if x.dim() else 0
     if in_dim != w.in_dim:
         raise RqError(-4, f"marlin_gemv: expected [{w.in_dim}], got {list(x.shape)}")
@@ -359,6 +394,9 @@ def _kv_quantize(t: torch.Tensor, mode: int):
 
 def _kv_quantize_pair(k: torch.Tensor, v: torch.Tensor, mode: int):
     """_kv_quantize of both, in the same launches where shape, type and device agree."""
+    r = (_rqc or _native()).kv_pair(k, v, mode, _KV_CODES[mode])
+    if r is not None:
+        return _done(r)
     if k.shape != v.shape or k.dtype != v.dtype or k.device != v.device:
         return (*_kv_quantize(k, mode), *_kv_quantize(v, mode))
     b, h, sd = _kv_dims(k)
@@ -381,6 +419,10 @@ def quantize_int8(t: torch.Tensor):
 
 
 def _kv_dequantize(q: torch.Tensor, scale: Optional[torch.Tensor], mode: int, target_dtype: torch.dtype):
+    if scale is not None:
+        r = (_rqc or _native()).kv_dequantize(q, scale, mode, target_dtype)
+        if r is not None:
+            return _done(r)
     b, h, sd = _kv_dims(q)
     out = torch.empty(q.shape, dtype=target_dtype, device=q.device)
     s = scale.reshape(-1).to(torch.float32).contiguous() if scale is not None else None
