@@ -239,6 +239,8 @@ int rq_embedding(const rq_weight *w, const uint32_t *ids, int64_t n_ids, float *
     (void)hipGetLastError();
     return set_error(RQ_E_ARG, "rq_embedding reads host ids and cannot be captured into a graph");
   }
+  rc = launch_gather_args(w, ids, n_ids, dev_out, s);
+  if (rc != RQ_E_UNSUPPORTED) return rc;
   WsLease ws(w->device, s);
   uint32_t *dids = static_cast<uint32_t *>(ws.get((size_t)n_ids * sizeof(uint32_t), &rc));
   if (!dids) return rc;

@@ -11,6 +11,8 @@
 //
 // Roofline: HBM-bound; per element the algorithmic traffic is the block bytes
 // per element read plus 4 bytes of f32 written.
+#include <string.h>
+
 #include "rq_internal.h"
 
 namespace rq {
@@ -256,6 +258,22 @@ __global__ __launch_bounds__(kThreads) void k_gather_rows(const uint8_t *__restr
   }
 }
 
+// The same for up to kIdArgs ids that travel in the kernel's arguments: one
+// workgroup row a row, its id one scalar load.  Bound: the call itself (about 3
+// us of kernel); the copy of the ids to the device that this saves took a blit
+// kernel of 3 us and as much of the host (512 rows of 896 from a Q8_0 table 8.5 -> 5.7 us).
+struct IdArgs {
+  uint32_t v[kIdArgs];
+};
+template <int QT>
+__global__ __launch_bounds__(kThreads) void k_gather_args(const uint8_t *__restrict__ data,
+                                                         const uint8_t *__restrict__ aux, uint32_t kq,
+                                                         float4 *__restrict__ out, const IdArgs ids) {
+  const uint64_t row = (uint64_t)ids.v[blockIdx.y] * kq;
+  const uint32_t q = blockIdx.x * kThreads + threadIdx.x;
+  if (q < kq) out[(uint64_t)blockIdx.y * kq + q] = quad_handle<QT>(data, aux, row + q);
+}
+
 // y[m, n] = x W^T for any shape and alignment (the shapes the fused kernels
 // do not take): one wave per weight row, the lanes striding over k, each
 // weight decoded exactly from its flat quad (the element picked from the
@@ -341,6 +359,11 @@ struct GatherK {
   static constexpr auto fn = k_gather_rows<QT>;
 };
 
+template <int QT>
+struct GatherArgsK {
+  static constexpr auto fn = k_gather_args<QT>;
+};
+
 int launch_dequant_weight(const rq_weight *w, float *out, hipStream_t s) {
   const uint64_t quads = (uint64_t)w->n * (uint64_t)w->k / 4;
   if (quads == 0) return RQ_OK;
@@ -354,6 +377,17 @@ int launch_gather_rows(const rq_weight *w, const uint32_t *dev_ids, int64_t n_id
   return by_qtype<GatherK>(w->qtype, dim3(grid_for((uint64_t)n_ids * (uint64_t)kq)), s, (const uint8_t *)w->data,
                            (const uint8_t *)(w->data + w->aux_off), dev_ids, n_ids, kq,
                            reinterpret_cast<float4 *>(out));
+}
+
+int launch_gather_args(const rq_weight *w, const uint32_t *host_ids, int64_t n_ids, float *out, hipStream_t s) {
+  if (n_ids == 0) return RQ_OK;
+  if (n_ids > kIdArgs || w->k / 4 > 0x7FFFFFFF) return RQ_E_UNSUPPORTED;
+  IdArgs ids = {};
+  memcpy(ids.v, host_ids, (size_t)n_ids * sizeof(uint32_t));
+  const uint32_t kq = (uint32_t)(w->k / 4);
+  return by_qtype<GatherArgsK>(w->qtype, dim3((kq + kThreads - 1) / kThreads, (unsigned)n_ids), s,
+                               (const uint8_t *)w->data, (const uint8_t *)(w->data + w->aux_off), kq,
+                               reinterpret_cast<float4 *>(out), ids);
 }
 
 int launch_linear_generic(const rq_weight *w, const void *x, int xtype, int64_t m, const Out &o, hipStream_t s) {

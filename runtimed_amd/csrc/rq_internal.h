@@ -233,6 +233,10 @@ int launch_dequant_weight(const rq_weight *w, float *out, hipStream_t s);
 // Rows dev_ids[0 .. n_ids) of a handle (every id < n, k % 4 == 0) as f32.
 int launch_gather_rows(const rq_weight *w, const uint32_t *dev_ids, int64_t n_ids, float *out,
                        hipStream_t s);
+// The same from host ids, at most kIdArgs of them (kernel arguments are 4 KB),
+// RQ_E_UNSUPPORTED otherwise.
+constexpr int kIdArgs = 512;
+int launch_gather_args(const rq_weight *w, const uint32_t *host_ids, int64_t n_ids, float *out, hipStream_t s);
 int launch_dequant_raw(int qtype, const uint8_t *src, uint64_t nblocks, float *out,
                        hipStream_t s);
 // Fused matmul on a handle (x 16-byte aligned); returns RQ_E_UNSUPPORTED
