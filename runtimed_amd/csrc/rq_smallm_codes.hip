@@ -493,8 +493,10 @@ int codes_launch(const rq_weight *const *w, int count, bool set, const float *x,
 
 // Plan: K split over S workgroups (up to 4) where few row tiles leave CUs idle
 // and there are 16 or more rows (or long rows); eight waves, one chunk a
-// batch; two row tiles a workgroup from 256 workgroups (a launch that would
-// fill the CUs more than once, or nearly); the activation slice in LDS from
+// batch; two row tiles a workgroup above 256 workgroups (a launch that would
+// fill the CUs more than once; 256 of them lose a CU's worth each: Q4_K 2 x 2048
+// x 2048 10.1 us against 7.7 on one, Q8_0 1024 x 3072 18.0 against 11.4, Q4_K
+// 4096 + 1024 x 4096 17.3 against 20.5); the activation slice in LDS from
 // 16 rows when it fits.  Graph-timed, 32 distinct Q4_K copies of the 0.5B
 // layer, us a launch, against the f32 matrix-core kernel (one weight) and the
 // two-limb set kernel (q/k/v, gate/up) -> this kernel:
@@ -546,7 +548,7 @@ int codes_plan(const rq_weight *const *w, int count, bool set, const float *x, i
   if (ws != nullptr && tiles <= WsLease::kCounters && tiles < 128 && !(w[0]->k <= 1024 && m <= 64) &&
       (m >= 16 || nk > 32))
     while (S < 4 && tiles * S * 2 <= 512 && nk >= 4 * S) S *= 2;
-  const int rt = tiles * S >= 256 ? 2 : 1;
+  const int rt = tiles * S > 256 ? 2 : 1;
   if (rt == 2) return codes_go<C, MT, 2>(w, count, set, x, m, o, s, ws, S);
   return codes_go<C, MT, 1>(w, count, set, x, m, o, s, ws, S);
 }
