@@ -291,7 +291,7 @@ static const void *aligned_x(const void *x, int xtype, int64_t m, int64_t k, hip
   return *rc ? nullptr : p;
 }
 
-// Whether a prefill call (m > 64) goes to the codes GEMM, which packs the
+// Whether a call goes to the codes GEMM, which packs the
 // activations in a launch of its own (4-8 us) and reads them in one launch for
 // all weights, or to the tiled kernels.  Graph-timed, codes GEMM against
 // tiled, us:
@@ -308,11 +308,33 @@ static const void *aligned_x(const void *x, int xtype, int64_t m, int64_t k, hip
 //     and long rows on few tiles (896 x 4864 at m = 65 / 512 22 / 30 against 29
 //     / 32, 4096 x 4096 at m = 65 23.5 against 26.7, 2048 x 2048 16.6 against
 //     13.9, 8192 x 2048 at m = 512 54 against 33) pay.
+// At most 64 rows (32 x 64 tiles up to 32): the small-M kernels read the
+// weights a lane its own row, which the vector cache serves one access a lane;
+// the codes GEMM reads them coalesced but pays the pack, so it takes the calls
+// with many weights.  f32 rows, small-M (m = 2, 3: VALU) against codes, us:
+//   m = 5 / 24: Q6_K 2048 x 8192 36.3 / 53.6 against 20.3 / 21.0, 4096 x 14336
+//     104 / 135 against 37 / 37, Q4_K 2 x 8192 x 2048 17.3 / 26.2 against 16.7 /
+//     17.3, 2 x 14336 x 4096 57 / 91 against 38 / 40, 4096 x 4096 16.6 / 25.4
+//     against 16.1 / 16.7, Q8_0 2 x 8192 x 2048 23.9 / 33.7 against 17.0 / 17.7;
+//     2 x 2048 x 2048 9.9 / 14.6 against 12.6 / 13.1, 2048 x 2048 6.7 / 8.8
+//     against 12.5 / 12.9
+//   m = 48 (64 x 64 tiles): 2 x 2048 x 2048 23.5 against 17.9, 2 x 8192 x 2048
+//     45.7 against 24.4, Q6_K 2048 x 8192 67.5 against 27.0, 2048 x 2048 15.5
+//     against 18.2
+//   m = 2 / 3: 2 x 8192 x 2048 15.1 / 34.8 against 16.7, 2 x 14336 x 4096 70 / 94
+//     against 38, Q6_K 2048 x 8192 14.2 / 17.4 against 20, 4096 x 14336 42.8 / 42.1
+//     against 35
+//   f16 rows as f32: 2 x 8192 x 2048 24.9 / 46.4 against 14.6 / 15.0.  bf16 rows
+//     (weights rounded to bf16 in the small-M kernel): 12.2 / 13.9 against 15.1 /
+//     15.7, Q6_K 2048 x 8192 29.6 / 33.0 against 18.1 / 18.4, m = 48 36 against 21.
 static bool codes_pay(const rq_weight *const *w, int count, int xtype, int64_t m) {
-  if (m <= 64) return false;
   const int64_t k = w[0]->k;
-  int64_t tiles = 0;
-  for (int j = 0; j < count; ++j) tiles += ((w[j]->n + 63) / 64) * ((m + 63) / 64);
+  int64_t tiles = 0, rows = 0;
+  for (int j = 0; j < count; ++j) tiles += ((w[j]->n + 63) / 64) * ((m + 63) / 64), rows += w[j]->n;
+  if (m <= 64) {
+    if (xtype == RQ_BF16) return m >= 3 && rows * k >= (int64_t)1 << 24 && (m > 32 || k >= 8192);
+    return m >= 2 && rows * k >= (m == 2 ? (int64_t)3 << 24 : (int64_t)1 << (m == 3 ? 25 : m <= 16 ? 24 : 23));
+  }
   if (xtype == RQ_BF16) return count > 1 ? tiles <= 400 : k >= 4096 && tiles <= 112;
   if (count > 1) return true;
   const bool kfmt = w[0]->qtype == RQ_Q4_K || w[0]->qtype == RQ_Q5_K || w[0]->qtype == RQ_Q6_K;
@@ -376,9 +398,10 @@ int rq_linear_multi(int count, const rq_weight *const *wts, const void *x, int x
     int j = i + 1;
     while (j < count && j - i < kMultiMax && wts[j]->qtype == wts[i]->qtype) ++j;
     for (int t = i; t < j; ++t) outs[t - i] = Out{ys[t], biases ? biases[t] : nullptr, ytype, btype};
-    rc = j - i == 1                                ? RQ_E_UNSUPPORTED
-         : codes_pay(wts + i, j - i, xtype, m) ? launch_linear_codes(wts + i, j - i, xa, xtype, m, outs, s, ws)
-                                                   : launch_linear_multi(wts + i, j - i, xa, xtype, m, outs, s, ws);
+    rc = RQ_E_UNSUPPORTED;
+    if (j - i > 1 && codes_pay(wts + i, j - i, xtype, m))
+      rc = launch_linear_codes(wts + i, j - i, xa, xtype, m, outs, s, ws);
+    if (j - i > 1 && rc == RQ_E_UNSUPPORTED) rc = launch_linear_multi(wts + i, j - i, xa, xtype, m, outs, s, ws);
     if (rc == RQ_E_UNSUPPORTED) {
       rc = RQ_OK;
       for (int t = i; t < j && !rc; ++t) rc = linear_one(wts[t], xa, xtype, m, outs[t - i], s, ws);
@@ -475,12 +498,13 @@ int rq_marlin_linear(const uint32_t *packed, const float *scales, int64_t n, int
   if (m == 0 || n == 0) return RQ_OK;
   if (!packed || !scales || !x || !y) return set_error(RQ_E_ARG, "null argument");
   hipStream_t s = as_stream(stream);
-  // The codes GEMM (which packs x in a launch of its own) from about 2^26
-  // multiply-adds (f32 x; 2^25.3 for 16-bit x, one matrix pass): an MLP of 2048
-  // / 8192 at m = 3 / 4 / 16 58.2 / 58.8 / 60.1 us against 51.8 / 62.7 / 179.6,
-  // 4096 / 14336 at m = 2 84.5 against 88.9, 512 / 1024 at m = 32 / 64 35.9 /
-  // 40.3 against 23.6 / 43.5.
-  if (m > 1 && (double)m * (double)n * (double)k >= (xtype == RQ_F32 ? 67.0e6 : 42.0e6)) {
+  // The codes GEMM (which packs x in a launch of its own) from about 4.2e7
+  // multiply-adds: f32, VALU against codes, 8192 x 2048 at m = 2 / 3 / 8 / 32 11.2
+  // / 15.1 / 32.5 / 124 against 13.0 / 13.0 / 12.9 / 13.4 us, 2048 x 2048 at m = 8
+  // / 16 9.4 / 17.3 against 12.6 / 13.3, 2048 x 1024 at m = 8 / 16 6.3 / 11.1
+  // against 9.7 / 9.7, 4096 x 14336 at m = 2 / 3 31.5 / 40.9 against 31.5 / 31.8;
+  // 1024 x 512 at m = 32 / 64 9.0 / 16.6 against 10.0 / 13.6.
+  if (m > 1 && (double)m * (double)n * (double)k >= 42.0e6) {
     int dev = 0;
     int rc = hip_check(hipGetDevice(&dev), "hipGetDevice");
     if (rc) return rc;

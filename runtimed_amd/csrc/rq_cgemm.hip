@@ -22,7 +22,7 @@
 // workgroup split K and meet once in LDS at the end.
 //
 // Product (k_cgemm): a wave owns a 64 x 64 tile of y over its share of K (2 x 2
-// MFMA tiles of 32 x 32), KG waves (8 at most) a workgroup.  Per chunk of 64
+// MFMA tiles of 32 x 32; 32 x 64 for at most 32 rows), KG waves (8 at most) a workgroup.  Per chunk of 64
 // inputs and weight row a lane loads its bytes of the row (the two lanes of a
 // row take the two 8-input halves of every 16-input step), makes four f16 B
 // operands of them, and sums S over a scale's run from zero; S joins the f32
@@ -663,13 +663,13 @@ __device__ __forceinline__ void cg_finish(float v, const SetEntry &en, const flo
 // VMEM stays where it is written; ALU, LDS and matrix work may move across.
 #define CG_PIN_LOADS() __builtin_amdgcn_sched_barrier(0x1 | 0x2 | 0x4 | 0x8 | 0x80 | 0x100 | 0x200)
 
-template <class D, int NL>
+template <class D, int NL, int MI>
 __global__ __launch_bounds__(512) void k_cgemm(const WeightSet set, const float *__restrict__ rs,
                                                const uint8_t *__restrict__ xp, const uint8_t *__restrict__ xsum,
                                                const int *__restrict__ rexp, const void *__restrict__ x, int xtype,
                                                int64_t m, int64_t k, int np, int tm, int S,
                                                float *__restrict__ part) {
-  // a staging region of 64 rows a wave, later KG tiles of 64 x 64 sums
+  // a staging region of 64 rows a wave, later KG tiles of 32 MI x 64 sums
   extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int KG = (int)(blockDim.x >> 6);
@@ -681,7 +681,7 @@ __global__ __launch_bounds__(512) void k_cgemm(const WeightSet set, const float 
   const int tile = unit / S, z = unit - tile * S;
   const SetEntry en = pick_entry(set, tile);
   const int lt = tile - en.g0, ntile = lt / tm, mtile = lt - ntile * tm;
-  const int n0 = 64 * ntile < en.n - 64 ? 64 * ntile : en.n - 64, m0 = 64 * mtile;
+  const int n0 = 64 * ntile < en.n - 64 ? 64 * ntile : en.n - 64, m0 = 32 * MI * mtile;
   D dec;
   if constexpr (D::MAP == MAP_MARLIN) {
     dec.stride = 16 * (int64_t)en.n;
@@ -692,18 +692,18 @@ __global__ __launch_bounds__(512) void k_cgemm(const WeightSet set, const float 
   const int lo = np * part_i / (KG * S), hi = np * (part_i + 1) / (KG * S);
   lds_u8 *const L = (lds_u8 *)lds + 64 * D::STRIDE * wave;
 
-  f32x16 acc[2][2];
+  f32x16 acc[MI][2];
 #pragma unroll
-  for (int i = 0; i < 2; ++i)
+  for (int i = 0; i < MI; ++i)
 #pragma unroll
     for (int j = 0; j < 2; ++j) acc[i][j] = (f32x16){0};
 
   if (lo < hi) {
-    const uint8_t *xa[2];
+    const uint8_t *xa[MI];
 #pragma unroll
-    for (int mi = 0; mi < 2; ++mi) xa[mi] = xp + (2 * (int64_t)mtile + mi) * (2 * np) * (NL * 4096);
+    for (int mi = 0; mi < MI; ++mi) xa[mi] = xp + (MI * (int64_t)mtile + mi) * (2 * np) * (NL * 4096);
     const uint32_t lo16 = 16u * lane;
-    u32x4 a[2][NL][4];
+    u32x4 a[MI][NL][4];
     typename D::Stage st;
     auto load_a = [&](int mi, int l, int s, int c) __attribute__((always_inline)) {
       a[mi][l][s] = ld16(xa[mi] + (int64_t)c * (NL * 4096) + (l * 4096 + s * 1024), lo16);
@@ -715,7 +715,7 @@ __global__ __launch_bounds__(512) void k_cgemm(const WeightSet set, const float 
 #pragma unroll
       for (int s = 0; s < 4; ++s)
 #pragma unroll
-        for (int mi = 0; mi < 2; ++mi) load_a(mi, l, s, 2 * lo);
+        for (int mi = 0; mi < MI; ++mi) load_a(mi, l, s, 2 * lo);
     CG_PIN_LOADS();
     // A chunk's matrix work; its A operands are reloaded for the chunk after
     // it (not LAST) as soon as the second column tile has used them.
@@ -731,12 +731,12 @@ __global__ __launch_bounds__(512) void k_cgemm(const WeightSet set, const float 
         dec.decode(L, ni, c, j, lane, b, d, mins[ni][c], dm[ni]);
         static_for<4 / D::GRP>([&](auto GG) __attribute__((always_inline)) {
           constexpr int s0 = decltype(GG)::value * D::GRP;
-          f32x16 S[2];
+          f32x16 S[MI];
           static_for<NL>([&](auto LL) __attribute__((always_inline)) {  // the small limb first
             constexpr int l = NL - 1 - decltype(LL)::value;
             static_for<D::GRP>([&](auto SS) __attribute__((always_inline)) {
               constexpr int s = s0 + decltype(SS)::value;
-              static_for<2>([&](auto MM) __attribute__((always_inline)) {
+              static_for<MI>([&](auto MM) __attribute__((always_inline)) {
                 constexpr int mi = decltype(MM)::value;
                 const f32x16 z = {0};
                 S[mi] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8, a[mi][l][s]), b[s],
@@ -748,7 +748,7 @@ __global__ __launch_bounds__(512) void k_cgemm(const WeightSet set, const float 
               });
             });
           });
-          static_for<2>([&](auto MM) __attribute__((always_inline)) {
+          static_for<MI>([&](auto MM) __attribute__((always_inline)) {
             constexpr int mi = decltype(MM)::value;
 #pragma unroll
             for (int r = 0; r < 16; ++r) {
@@ -767,10 +767,10 @@ __global__ __launch_bounds__(512) void k_cgemm(const WeightSet set, const float 
         dec.issue(st, j + 1, lane);
         CG_PIN_LOADS();
       }
-      u32x4 xs[2];
+      u32x4 xs[MI];
       if constexpr (D::MINS) {
 #pragma unroll
-        for (int mi = 0; mi < 2; ++mi) xs[mi] = ld16(xsum + ((2 * (int64_t)mtile + mi) * np + j) * 1024, lo16);
+        for (int mi = 0; mi < MI; ++mi) xs[mi] = ld16(xsum + ((MI * (int64_t)mtile + mi) * np + j) * 1024, lo16);
         CG_PIN_LOADS();
       }
       chunk(j, std::integral_constant<int, 0>{}, std::false_type{});
@@ -783,7 +783,7 @@ __global__ __launch_bounds__(512) void k_cgemm(const WeightSet set, const float 
           constexpr int ni = decltype(NI)::value;
           const bool h0 = lane < 32;
           const u32x4 mb = {mins[ni][0], mins[ni][1], h0 ? mins[ni][0] : 0u, h0 ? mins[ni][1] : 0u};
-          static_for<2>([&](auto MM) __attribute__((always_inline)) {
+          static_for<MI>([&](auto MM) __attribute__((always_inline)) {
             constexpr int mi = decltype(MM)::value;
             const f32x16 z = {0};
             const f32x16 M = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(cg_bf16x8, xs[mi]),
@@ -801,45 +801,47 @@ __global__ __launch_bounds__(512) void k_cgemm(const WeightSet set, const float 
   // The waves' tiles summed in wave order.  Slot q of a tile: MFMA tile
   // q / 16 (32 x 32: row half q / 32, column half (q / 16) % 2), register
   // q % 16; a wave takes every KG-th slot, two rows of 32 outputs each.
+  constexpr int TS = 2048 * MI;  // sums of a tile
   float *const red = reinterpret_cast<float *>(lds);
   __syncthreads();  // every wave's staging reads are done
-  float *mine = red + 4096 * wave + lane;
+  float *mine = red + TS * wave + lane;
 #pragma unroll
-  for (int mi = 0; mi < 2; ++mi)
+  for (int mi = 0; mi < MI; ++mi)
 #pragma unroll
     for (int ni = 0; ni < 2; ++ni)
 #pragma unroll
       for (int r = 0; r < 16; ++r) mine[((2 * mi + ni) * 16 + r) * 64] = acc[mi][ni][r];
   __syncthreads();
-  for (int q = wave; q < 64; q += KG) {
+  for (int q = wave; q < 32 * MI; q += KG) {
     float v = red[64 * q + lane];
-    for (int w = 1; w < KG; ++w) v += red[4096 * w + 64 * q + lane];
+    for (int w = 1; w < KG; ++w) v += red[TS * w + 64 * q + lane];
     const int64_t row = m0 + 32 * (q >> 5) + 8 * ((q & 15) >> 2) + (q & 3) + 4 * (lane >> 5);
     const int col = n0 + 32 * ((q >> 4) & 1) + (lane & 31);
     if (row < m) {
-      if (part) part[((int64_t)tile * S + z) * 4096 + 64 * q + lane] = v;
+      if (part) part[((int64_t)tile * S + z) * TS + 64 * q + lane] = v;
       else cg_finish<D>(v, en, rs, rexp, x, xtype, row, col, k);
     }
   }
 }
 
 // Split K: the S slices of every tile added in order, one thread an output.
-template <class D>
+template <class D, int MI>
 __global__ __launch_bounds__(256) void k_cg_sum(const WeightSet set, const float *__restrict__ rs,
                                                 const float *__restrict__ part, const int *__restrict__ rexp,
                                                 const void *__restrict__ x, int xtype, int64_t m, int64_t k, int tm,
                                                 int S) {
-  const int tile = (int)blockIdx.x >> 4, q = 4 * ((int)blockIdx.x & 15) + (int)(threadIdx.x >> 6);
+  constexpr int WG = 8 * MI, TS = 2048 * MI;  // workgroups a tile, sums of a tile
+  const int tile = (int)blockIdx.x / WG, q = 4 * ((int)blockIdx.x % WG) + (int)(threadIdx.x >> 6);
   const int lane = threadIdx.x & 63;
   const SetEntry en = pick_entry(set, tile);
   const int lt = tile - en.g0, ntile = lt / tm, mtile = lt - ntile * tm;
-  const int64_t row = 64 * (int64_t)mtile + 32 * (q >> 5) + 8 * ((q & 15) >> 2) + (q & 3) + 4 * (lane >> 5);
+  const int64_t row = 32 * MI * (int64_t)mtile + 32 * (q >> 5) + 8 * ((q & 15) >> 2) + (q & 3) + 4 * (lane >> 5);
   const int n0 = 64 * ntile < en.n - 64 ? 64 * ntile : en.n - 64;
   const int col = n0 + 32 * ((q >> 4) & 1) + (lane & 31);
   if (row >= m) return;
-  const float *p = part + (int64_t)tile * S * 4096 + 64 * q + lane;
+  const float *p = part + (int64_t)tile * S * TS + 64 * q + lane;
   float v = p[0];
-  for (int z = 1; z < S; ++z) v += p[4096 * z];
+  for (int z = 1; z < S; ++z) v += p[TS * z];
   cg_finish<D>(v, en, rs, rexp, x, xtype, row, col, k);
 }
 
@@ -866,64 +868,73 @@ bool lds_allow(size_t bytes) {
 // pair takes about 1 + w / 8 half-units (measured, eight waves: 3.3 - 4.9 us a
 // pair with one limb, 3.6 - 6.6 with two), a round of workgroups about 4 us
 // beside its pairs (first loads, sum over the waves, stores), the second
-// kernel 3 us and its reads (16 KB a tile and slice at 3.5 TB/s).
+// kernel 3 us and its reads (16 KB a tile and slice at 3.5 TB/s).  On
+// tiles of 32 rows a pair waits on its loads rather than on the matrix cores:
+// 1.5 + w / 4 us (m = 5, with the pack: 2 x
+// 8192 x 2048 16.7 us on eight waves a tile, 2 x 14336 x 4096 38.3 on four and
+// 42.3 on eight, 2048 x 8192 20.3 / 22.6 / 28.3 / 38.7 on 8 / 4 / 2 / 1 slices).
 struct Plan {
   int kg, S;
 };
-Plan cg_plan(int64_t tiles, int np, int nl) {
+Plan cg_plan(int64_t tiles, int np, int nl, int mi) {
   Plan best{1, 1};
   double cost = 1e30;
   for (int S = 1; S <= 8; S *= 2) {
     for (int kg = 1; kg <= 8; ++kg) {
       if (kg * S > np && kg * S > 1) continue;
-      const int64_t slots = 256 * (8 / kg), wgs = tiles * S, rounds = (wgs + slots - 1) / slots;
-      const int64_t per_cu = (wgs + 255) / 256 < 8 / kg ? (wgs + 255) / 256 : 8 / kg;
-      const double unit = (nl == 2 ? 2.5 : 2.0) * (1.0 + (double)(per_cu * kg) / 8.0);
+      const int res = 8 / kg;  // workgroups a CU holds
+      const int64_t slots = 256 * res, wgs = tiles * S, rounds = (wgs + slots - 1) / slots;
+      const int64_t per_cu = (wgs + 255) / 256 < res ? (wgs + 255) / 256 : res;
+      const double unit = mi == 1 ? (nl == 2 ? 1.0 : 0.85) * (1.5 + 0.25 * (double)(per_cu * kg))
+                                  : (nl == 2 ? 2.5 : 2.0) * (1.0 + (double)(per_cu * kg) / 8.0);
       const double c = (double)rounds * (4.0 + unit * (double)((np + kg * S - 1) / (kg * S))) +
-                       (S > 1 ? 3.0 + (double)wgs * 16384.0 / 3.5e6 : 0.0);
+                       (S > 1 ? 3.0 + (double)wgs * 8192.0 * mi / 3.5e6 : 0.0);
       if (c <= cost) cost = c, best = Plan{kg, S};
     }
   }
   return best;
 }
 
-constexpr size_t cg_lds(int kg, int stride) {
-  const size_t a = (size_t)kg * 16384, b = (size_t)kg * 64 * stride;
+constexpr size_t cg_lds(int kg, int mi, int stride) {
+  const size_t a = (size_t)kg * 8192 * mi, b = (size_t)kg * 64 * stride;
   return a > b ? a : b;
 }
 
-template <class D, int NL>
+template <class D, int NL, int MI>
 int go(const WeightSet &set, int64_t tiles, const float *rs, const uint8_t *xp, const uint8_t *xsum, const int *rexp,
        const void *x, int xtype, int64_t m, int64_t k, int np, hipStream_t s, WsLease &ws) {
-  const Plan plan = cg_plan(tiles, np, NL);
+  const Plan plan = cg_plan(tiles, np, NL, MI);
   const int kg = plan.kg;
   int S = plan.S;
   float *part = nullptr;
   if (S > 1) {
     int rc = RQ_OK;
-    part = static_cast<float *>(ws.get((size_t)tiles * S * 16384, &rc, true));
+    part = static_cast<float *>(ws.get((size_t)tiles * S * 8192 * MI, &rc, true));
     if (!part) S = 1;
   }
-  const size_t lds = cg_lds(kg, D::STRIDE);
-  if (!lds_allow<&k_cgemm<D, NL>>(lds)) return RQ_E_UNSUPPORTED;
-  const int tm = (int)((m + 63) / 64);
-  hipLaunchKernelGGL((k_cgemm<D, NL>), dim3((unsigned)(tiles * S)), dim3(64 * kg), lds, s, set, rs, xp, xsum, rexp, x,
+  const size_t lds = cg_lds(kg, MI, D::STRIDE);
+  if (!lds_allow<&k_cgemm<D, NL, MI>>(lds)) return RQ_E_UNSUPPORTED;
+  const int tm = (int)((m + 32 * MI - 1) / (32 * MI));
+  hipLaunchKernelGGL((k_cgemm<D, NL, MI>), dim3((unsigned)(tiles * S)), dim3(64 * kg), lds, s, set, rs, xp, xsum, rexp, x,
                      xtype, m, k, np, tm, S, part);
   int rc = last_launch("codes gemm");
   if (!rc && S > 1) {
-    hipLaunchKernelGGL((k_cg_sum<D>), dim3((unsigned)(tiles * 16)), dim3(256), 0, s, set, rs, part, rexp, x, xtype, m,
+    hipLaunchKernelGGL((k_cg_sum<D, MI>), dim3((unsigned)(tiles * 8 * MI)), dim3(256), 0, s, set, rs, part, rexp, x, xtype, m,
                        k, tm, S);
     rc = last_launch("codes gemm sum");
   }
   return rc;
 }
 
+// Rows packed for m rows of x: whole tiles of 32 (m <= 32) or 64.
+int64_t cg_rows(int64_t m) { return m <= 32 ? 32 : (m + 63) / 64 * 64; }
+
 // One or two rows a workgroup where that many workgroups are needed to fill
 // the chip, else four (wider consecutive stores).
 template <int XT, int NL, int MAP, bool SUMS>
 int pack(const void *x, int64_t m, int64_t k, int np, uint8_t *xp, uint8_t *xsum, int *rexp, hipStream_t s) {
   const bool vec = k % 8 == 0 && reinterpret_cast<uintptr_t>(x) % 16 == 0;
-  const int64_t rows = (m + 63) / 64 * 64;
+  const int64_t rows = cg_rows(m);
 #define RQ_PACK(RW, B)                                                                                            \
   hipLaunchKernelGGL((k_cg_pack<XT, NL, MAP, SUMS, RW, B>), dim3((unsigned)(rows / RW)), dim3(kPackThreads), 0, s, \
                      x, m, k, np, vec, xp, xsum, rexp)
@@ -941,16 +952,16 @@ int pack(const void *x, int64_t m, int64_t k, int np, uint8_t *xp, uint8_t *xsum
   return last_launch("activation pack");
 }
 
-template <int NL>
+template <int NL, int MI>
 int by_type(int qtype, const WeightSet &set, int64_t tiles, const uint8_t *xp, const uint8_t *xsum, const int *rexp,
             const void *x, int xtype, int64_t m, int64_t k, int np, hipStream_t s, WsLease &ws) {
   switch (qtype) {
-    case RQ_Q4_K: return go<CgK4<false>, NL>(set, tiles, nullptr, xp, xsum, rexp, x, xtype, m, k, np, s, ws);
-    case RQ_Q5_K: return go<CgK4<true>, NL>(set, tiles, nullptr, xp, xsum, rexp, x, xtype, m, k, np, s, ws);
-    case RQ_Q6_K: return go<CgQ6K, NL>(set, tiles, nullptr, xp, xsum, rexp, x, xtype, m, k, np, s, ws);
-    case RQ_Q8_0: return go<CgQ8, NL>(set, tiles, nullptr, xp, xsum, rexp, x, xtype, m, k, np, s, ws);
-    case RQ_Q4_0: return go<CgQx0<false>, NL>(set, tiles, nullptr, xp, xsum, rexp, x, xtype, m, k, np, s, ws);
-    case RQ_Q5_0: return go<CgQx0<true>, NL>(set, tiles, nullptr, xp, xsum, rexp, x, xtype, m, k, np, s, ws);
+    case RQ_Q4_K: return go<CgK4<false>, NL, MI>(set, tiles, nullptr, xp, xsum, rexp, x, xtype, m, k, np, s, ws);
+    case RQ_Q5_K: return go<CgK4<true>, NL, MI>(set, tiles, nullptr, xp, xsum, rexp, x, xtype, m, k, np, s, ws);
+    case RQ_Q6_K: return go<CgQ6K, NL, MI>(set, tiles, nullptr, xp, xsum, rexp, x, xtype, m, k, np, s, ws);
+    case RQ_Q8_0: return go<CgQ8, NL, MI>(set, tiles, nullptr, xp, xsum, rexp, x, xtype, m, k, np, s, ws);
+    case RQ_Q4_0: return go<CgQx0<false>, NL, MI>(set, tiles, nullptr, xp, xsum, rexp, x, xtype, m, k, np, s, ws);
+    case RQ_Q5_0: return go<CgQx0<true>, NL, MI>(set, tiles, nullptr, xp, xsum, rexp, x, xtype, m, k, np, s, ws);
     default: return RQ_E_UNSUPPORTED;
   }
 }
@@ -967,7 +978,7 @@ Pack pack_bytes(int64_t rows, int np, int nl) {
 constexpr size_t kPackMax = 128u << 20;
 
 int64_t slice_rows(int64_t m, int np, int nl) {
-  int64_t rows = (m + 63) / 64 * 64;
+  int64_t rows = cg_rows(m);
   while (rows > 64 && pack_bytes(rows, np, nl).total() > kPackMax) rows = (rows / 2 + 63) / 64 * 64;
   return rows;
 }
@@ -1002,7 +1013,8 @@ int launch_linear_codes(const rq_weight *const *w, int count, const void *x, int
       os[j] = o[j];
       os[j].y = static_cast<uint8_t *>(o[j].y) + (size_t)r0 * (size_t)w[j]->n * (o[j].ytype == RQ_F32 ? 4 : 2);
     }
-    const int64_t tm = (mm + 63) / 64;
+    const bool few = mm <= 32;
+    const int64_t tm = few ? 1 : (mm + 63) / 64;
     WeightSet set;
     int64_t tiles = 0;
     rc = fill_set(set, w, count, os, [&](const rq_weight *wj) { return tm * ((wj->n + 63) / 64); }, &tiles);
@@ -1015,8 +1027,10 @@ int launch_linear_codes(const rq_weight *const *w, int count, const void *x, int
     else RQ_CG_PACK(RQ_F16, 1);
 #undef RQ_CG_PACK
     if (rc) return rc;
-    rc = nl == 2 ? by_type<2>(w[0]->qtype, set, tiles, xp, xsum, rexp, xs, xtype, mm, k, np, s, ws)
-                 : by_type<1>(w[0]->qtype, set, tiles, xp, xsum, rexp, xs, xtype, mm, k, np, s, ws);
+#define RQ_CG_GO(NL, MI) by_type<NL, MI>(w[0]->qtype, set, tiles, xp, xsum, rexp, xs, xtype, mm, k, np, s, ws)
+    if (few) rc = nl == 2 ? RQ_CG_GO(2, 1) : RQ_CG_GO(1, 1);
+    else rc = nl == 2 ? RQ_CG_GO(2, 2) : RQ_CG_GO(1, 2);
+#undef RQ_CG_GO
     if (rc) return rc;
   }
   return RQ_OK;
@@ -1036,7 +1050,8 @@ int launch_marlin_codes(const uint32_t *packed, const float *scales, int64_t n, 
   for (int64_t r0 = 0; r0 < m; r0 += rows) {
     const int64_t mm = m - r0 < rows ? m - r0 : rows;
     const void *xs = static_cast<const uint8_t *>(x) + (size_t)r0 * (size_t)k * xb;
-    const int64_t tiles = (mm + 63) / 64 * ((n + 63) / 64);
+    const bool few = mm <= 32;
+    const int64_t tiles = (few ? 1 : (mm + 63) / 64) * ((n + 63) / 64);
     if (tiles > 0x3FFFFFF) return RQ_E_UNSUPPORTED;
     WeightSet set = {};
     set.w[0] = reinterpret_cast<const uint8_t *>(packed);
@@ -1050,8 +1065,10 @@ int launch_marlin_codes(const uint32_t *packed, const float *scales, int64_t n, 
     else if (xtype == RQ_BF16) rc = pack<RQ_BF16, 1, MAP_MARLIN, false>(xs, mm, k, np, xp, nullptr, rexp, s);
     else rc = pack<RQ_F16, 1, MAP_MARLIN, false>(xs, mm, k, np, xp, nullptr, rexp, s);
     if (rc) return rc;
-    rc = nl == 2 ? go<CgMarlin, 2>(set, tiles, scales, xp, nullptr, rexp, xs, xtype, mm, k, np, s, ws)
-                 : go<CgMarlin, 1>(set, tiles, scales, xp, nullptr, rexp, xs, xtype, mm, k, np, s, ws);
+#define RQ_CG_GO(NL, MI) go<CgMarlin, NL, MI>(set, tiles, scales, xp, nullptr, rexp, xs, xtype, mm, k, np, s, ws)
+    if (few) rc = nl == 2 ? RQ_CG_GO(2, 1) : RQ_CG_GO(1, 1);
+    else rc = nl == 2 ? RQ_CG_GO(2, 2) : RQ_CG_GO(1, 2);
+#undef RQ_CG_GO
     if (rc) return rc;
   }
   return RQ_OK;
