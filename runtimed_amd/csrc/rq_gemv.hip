@@ -1019,6 +1019,13 @@ int launch_linear_multi(const rq_weight *const *w, int count, const void *x, int
     return rc != RQ_E_UNSUPPORTED ? rc : launch_linear_smallm_set(w, count, x, xtype, m, o, s, &ws);
   }
   if (m != 1 && m != 2) return RQ_E_UNSUPPORTED;
+  // Long Q4_K rows on many rows each: the matrix-core GEMV that each of them
+  // would take alone, in one launch.
+  if (m == 1 && qt == RQ_Q4_K && k > 64 * 32) {
+    for (int j = 0; j < count; ++j)
+      if (w[j]->n < 4096) return RQ_E_UNSUPPORTED;
+    return launch_gemv_mx_set(w, count, x, xtype, o, s);
+  }
   switch (qt) {
     case RQ_Q4_K: return k % 64 ? RQ_E_UNSUPPORTED : run_seg_set<FmtQ4K>(w, count, x, xtype, m, o, s);
     case RQ_Q6_K: return k % 128 ? RQ_E_UNSUPPORTED : run_seg_set<FmtQ6K>(w, count, x, xtype, m, o, s);

@@ -77,15 +77,15 @@ __device__ __forceinline__ mx_bf16x8 b_frag(uint32_t c0, uint32_t c1) {
   return __builtin_bit_cast(mx_bf16x8, v);
 }
 
-__global__ __launch_bounds__(1024) void k_gemv_mx(const uint8_t *__restrict__ w, const void *__restrict__ x,
-                                                  int xtype, const Out o, int64_t n, int64_t k) {
-  extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
+// Rows 32 tile .. 32 tile + 31 of one weight.
+__device__ __forceinline__ void mx_tile(const uint8_t *__restrict__ w, const void *__restrict__ x, int xtype,
+                                        const Out &o, int64_t n, int64_t k, int tile, uint8_t *lds) {
   const int tid = threadIdx.x, lane = tid & 63;
   const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int waves = (int)(blockDim.x >> 6);
   const int wr = lane & 31, h = lane >> 5;
   const uint32_t rstride = (uint32_t)(k >> 8) * 144u;  // bytes a row (the whole matrix is < 2 GB)
-  const int64_t row0 = (int64_t)blockIdx.x * 32;
+  const int64_t row0 = (int64_t)tile * 32;
   // Last row of this tile that exists (the last tile may be partial).
   const int rowcap = __builtin_amdgcn_readfirstlane((int)(n - row0 < 32 ? n - row0 - 1 : 31));
 
@@ -239,6 +239,20 @@ __global__ __launch_bounds__(1024) void k_gemv_mx(const uint8_t *__restrict__ w,
     for (int i = 0; i < waves; ++i) v += red[32 * i + tid];
     store_linear(o, 0, n, row0 + tid, v);
   }
+}
+
+__global__ __launch_bounds__(1024) void k_gemv_mx(const uint8_t *__restrict__ w, const void *__restrict__ x,
+                                                  int xtype, const Out o, int64_t n, int64_t k) {
+  extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
+  mx_tile(w, x, xtype, o, n, k, (int)blockIdx.x, lds);
+}
+
+// Several weights sharing x (gate / up of one layer) in one grid.
+__global__ __launch_bounds__(1024) void k_gemv_mx_set(const WeightSet set, const void *__restrict__ x, int xtype,
+                                                      int64_t k) {
+  extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
+  const SetEntry e = pick_entry(set, (int)blockIdx.x);
+  mx_tile(e.w, x, xtype, e.o, e.n, k, (int)blockIdx.x - e.g0, lds);
 }
 
 // ---- Q6_K (dequant_k.rs:94-125) ----
@@ -417,26 +431,44 @@ __global__ __launch_bounds__(1024) void k_gemv_mx6(const uint8_t *__restrict__ w
 
 }  // namespace
 
-int launch_gemv_mx(const rq_weight *wt, const void *x, int xtype, const Out &o, hipStream_t s) {
+static bool mx_takes(const rq_weight *wt, const void *x) {
   const int64_t n = wt->n, k = wt->k;
-  if (wt->qtype != RQ_Q4_K || k % (256 * kMxSb) != 0 || k > kMxMaxK || n < 32) return RQ_E_UNSUPPORTED;
-  if (reinterpret_cast<uintptr_t>(x) % 16 != 0) return RQ_E_UNSUPPORTED;
-  // 32-bit byte offsets inside the matrix.
-  if ((uint64_t)n * (uint64_t)(k / 256) * 144u >= (1ull << 31)) return RQ_E_UNSUPPORTED;
-  const int64_t grid = (n + 31) / 32;
+  return wt->qtype == RQ_Q4_K && k % (256 * kMxSb) == 0 && k <= kMxMaxK && n >= 32 &&
+         reinterpret_cast<uintptr_t>(x) % 16 == 0 &&
+         // 32-bit byte offsets inside the matrix.
+         (uint64_t)n * (uint64_t)(k / 256) * 144u < (1ull << 31);
+}
+
+// Above 64 KB of dynamic LDS (k > 4096) a kernel asks for it once.
+template <auto KERNEL>
+static bool mx_lds_allow(size_t lds) {
+  if (lds <= 65536) return true;
+  static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void *>(KERNEL),
+                                                     hipFuncAttributeMaxDynamicSharedMemorySize,
+                                                     (int)mx_lds_bytes(kMxMaxK));
+  if (attr != hipSuccess) (void)hipGetLastError();
+  return attr == hipSuccess;
+}
+
+int launch_gemv_mx(const rq_weight *wt, const void *x, int xtype, const Out &o, hipStream_t s) {
+  const size_t lds = mx_lds_bytes(wt->k);
+  if (!mx_takes(wt, x) || !mx_lds_allow<&k_gemv_mx>(lds)) return RQ_E_UNSUPPORTED;
+  hipLaunchKernelGGL(k_gemv_mx, dim3((unsigned)((wt->n + 31) / 32)), dim3((unsigned)(wt->k / 8)), lds, s, wt->data, x,
+                     xtype, o, wt->n, wt->k);
+  return hipGetLastError() == hipSuccess ? RQ_OK : set_error(RQ_E_DEVICE, "gemv launch failed");
+}
+
+int launch_gemv_mx_set(const rq_weight *const *w, int count, const void *x, int xtype, const Out *o, hipStream_t s) {
+  const int64_t k = w[0]->k;
+  for (int j = 0; j < count; ++j)
+    if (w[j]->k != k || !mx_takes(w[j], x)) return RQ_E_UNSUPPORTED;
   const size_t lds = mx_lds_bytes(k);
-  if (lds > 65536) {
-    // Above 64 KB of dynamic LDS (k > 4096) the kernel asks for it once.
-    static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void *>(&k_gemv_mx),
-                                                       hipFuncAttributeMaxDynamicSharedMemorySize,
-                                                       (int)mx_lds_bytes(kMxMaxK));
-    if (attr != hipSuccess) {
-      (void)hipGetLastError();
-      return RQ_E_UNSUPPORTED;
-    }
-  }
-  hipLaunchKernelGGL(k_gemv_mx, dim3((unsigned)grid), dim3((unsigned)(k / 8)), lds, s, wt->data, x, xtype, o, n,
-                     k);
+  if (!mx_lds_allow<&k_gemv_mx_set>(lds)) return RQ_E_UNSUPPORTED;
+  WeightSet set;
+  int64_t total = 0;
+  const int rc = fill_set(set, w, count, o, [](const rq_weight *wj) { return (wj->n + 31) / 32; }, &total);
+  if (rc) return rc;
+  hipLaunchKernelGGL(k_gemv_mx_set, dim3((unsigned)total), dim3((unsigned)(k / 8)), lds, s, set, x, xtype, k);
   return hipGetLastError() == hipSuccess ? RQ_OK : set_error(RQ_E_DEVICE, "gemv launch failed");
 }
 

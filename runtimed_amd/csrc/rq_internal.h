@@ -247,6 +247,8 @@ int launch_linear_fused(const rq_weight *w, const void *x, int xtype, int64_t m,
 // M = 1 Q4_K GEMV on the matrix cores (k % 512 == 0, k <= 8192, x 16-byte
 // aligned); RQ_E_UNSUPPORTED for other shapes.
 int launch_gemv_mx(const rq_weight *w, const void *x, int xtype, const Out &o, hipStream_t s);
+// The same for several weights of one k sharing x in one launch.
+int launch_gemv_mx_set(const rq_weight *const *w, int count, const void *x, int xtype, const Out *o, hipStream_t s);
 // The same for Q6_K (k % 512 == 0, k <= 8192).
 int launch_gemv_mx6(const rq_weight *w, const void *x, int xtype, const Out &o, hipStream_t s);
 // One launch for several weights of one format sharing x (count <= kMultiMax,
