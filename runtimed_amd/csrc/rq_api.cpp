@@ -343,8 +343,8 @@ static bool codes_pay(const rq_weight *const *w, int count, int xtype, int64_t m
 
 // One weight: the fused kernels, or the generic one for shapes they do not take.
 static int linear_one(const rq_weight *w, const void *xa, int xtype, int64_t m, const Out &o, hipStream_t s,
-                      WsLease &ws) {
-  int rc = codes_pay(&w, 1, xtype, m) ? launch_linear_codes(&w, 1, xa, xtype, m, &o, s, ws) : RQ_E_UNSUPPORTED;
+                      WsLease &ws, CodesPack *pack = nullptr) {
+  int rc = codes_pay(&w, 1, xtype, m) ? launch_linear_codes(&w, 1, xa, xtype, m, &o, s, ws, pack) : RQ_E_UNSUPPORTED;
   if (rc == RQ_E_UNSUPPORTED) rc = launch_linear_fused(w, xa, xtype, m, o, s, ws);
   if (rc == RQ_E_UNSUPPORTED) rc = launch_linear_generic(w, xa, xtype, m, o, s);
   return rc;
@@ -393,6 +393,10 @@ int rq_linear_multi(int count, const rq_weight *const *wts, const void *x, int x
   const void *xa = aligned_x(x, xtype, m, k, s, ws, &rc);
   if (!xa) return rc;
   Out outs[kMultiMax];
+  // Runs of several formats share one pack of x (q / k in Q4_K, v in Q6_K of
+  // 512 rows of 2048: 5 us less).
+  CodesPack pack;
+  for (int i = 0; i < count; ++i) pack.sums |= wts[i]->qtype == RQ_Q4_K || wts[i]->qtype == RQ_Q5_K;
   for (int i = 0; i < count;) {
     // A run of consecutive weights of one format (at most kMultiMax).
     int j = i + 1;
@@ -400,11 +404,11 @@ int rq_linear_multi(int count, const rq_weight *const *wts, const void *x, int x
     for (int t = i; t < j; ++t) outs[t - i] = Out{ys[t], biases ? biases[t] : nullptr, ytype, btype};
     rc = RQ_E_UNSUPPORTED;
     if (j - i > 1 && codes_pay(wts + i, j - i, xtype, m))
-      rc = launch_linear_codes(wts + i, j - i, xa, xtype, m, outs, s, ws);
+      rc = launch_linear_codes(wts + i, j - i, xa, xtype, m, outs, s, ws, &pack);
     if (j - i > 1 && rc == RQ_E_UNSUPPORTED) rc = launch_linear_multi(wts + i, j - i, xa, xtype, m, outs, s, ws);
     if (rc == RQ_E_UNSUPPORTED) {
       rc = RQ_OK;
-      for (int t = i; t < j && !rc; ++t) rc = linear_one(wts[t], xa, xtype, m, outs[t - i], s, ws);
+      for (int t = i; t < j && !rc; ++t) rc = linear_one(wts[t], xa, xtype, m, outs[t - i], s, ws, &pack);
     }
     if (rc) return rc;
     i = j;

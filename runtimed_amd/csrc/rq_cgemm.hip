@@ -986,7 +986,7 @@ int64_t slice_rows(int64_t m, int np, int nl) {
 }  // namespace
 
 int launch_linear_codes(const rq_weight *const *w, int count, const void *x, int xtype, int64_t m, const Out *o,
-                        hipStream_t s, WsLease &ws) {
+                        hipStream_t s, WsLease &ws, CodesPack *shared) {
   const int64_t k = w[0]->k;
   if (count < 1 || count > kMultiMax || m < 1 || k % 128 != 0 || k > (1 << 20) ||
       reinterpret_cast<uintptr_t>(x) % 16 != 0)
@@ -1000,11 +1000,15 @@ int launch_linear_codes(const rq_weight *const *w, int count, const void *x, int
   const int64_t rows = slice_rows(m, np, nl);
   const Pack pb = pack_bytes(rows, np, nl);
   int rc = RQ_OK;
-  uint8_t *xp = static_cast<uint8_t *>(ws.get(pb.total(), &rc, true));
+  const bool mins = w[0]->qtype == RQ_Q4_K || w[0]->qtype == RQ_Q5_K;
+  // One slice only: a later slice overwrites the pack.
+  if (rows < m) shared = nullptr;
+  const bool packed = shared && shared->xp && (shared->sums || !mins);
+  const bool sums = mins || (shared && shared->sums);
+  uint8_t *xp = packed ? const_cast<uint8_t *>(shared->xp) : static_cast<uint8_t *>(ws.get(pb.total(), &rc, true));
   if (!xp) return RQ_E_UNSUPPORTED;
   uint8_t *xsum = xp + pb.limbs;
   int *rexp = reinterpret_cast<int *>(xsum + pb.sums);
-  const bool sums = w[0]->qtype == RQ_Q4_K || w[0]->qtype == RQ_Q5_K;
   for (int64_t r0 = 0; r0 < m; r0 += rows) {
     const int64_t mm = m - r0 < rows ? m - r0 : rows;
     const void *xs = static_cast<const uint8_t *>(x) + (size_t)r0 * (size_t)k * xb;
@@ -1022,11 +1026,16 @@ int launch_linear_codes(const rq_weight *const *w, int count, const void *x, int
 #define RQ_CG_PACK(XT, NL)                                                                          \
   rc = sums ? pack<XT, NL, MAP_GGUF, true>(xs, mm, k, np, xp, xsum, rexp, s)                        \
             : pack<XT, NL, MAP_GGUF, false>(xs, mm, k, np, xp, xsum, rexp, s)
-    if (xtype == RQ_F32) RQ_CG_PACK(RQ_F32, 2);
+    if (packed) rc = RQ_OK;
+    else if (xtype == RQ_F32) RQ_CG_PACK(RQ_F32, 2);
     else if (xtype == RQ_BF16) RQ_CG_PACK(RQ_BF16, 1);
     else RQ_CG_PACK(RQ_F16, 1);
 #undef RQ_CG_PACK
     if (rc) return rc;
+    if (shared && !packed) {
+      shared->xp = xp;
+      shared->sums = sums;
+    }
 #define RQ_CG_GO(NL, MI) by_type<NL, MI>(w[0]->qtype, set, tiles, xp, xsum, rexp, xs, xtype, mm, k, np, s, ws)
     if (few) rc = nl == 2 ? RQ_CG_GO(2, 1) : RQ_CG_GO(1, 1);
     else rc = nl == 2 ? RQ_CG_GO(2, 2) : RQ_CG_GO(1, 2);

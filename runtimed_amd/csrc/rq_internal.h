@@ -292,8 +292,16 @@ int launch_linear_smallm_f32_slices(const rq_weight *wt, const void *x, int xtyp
 // sharing x (k % 64 == 0, x 16-byte aligned): the weights' integer codes on
 // the f16 matrix cores.  RQ_E_UNSUPPORTED for other shapes, or where the
 // packed activations find no scratch.
+// `shared` (null: none) lives for one entry-point call on one x: the first
+// launch leaves its packed activations there, with the sums the K formats need
+// if `sums` asks for them, and the launches on weights of other formats read
+// them (in the workspace of the same lease, so in stream order).
+struct CodesPack {
+  bool sums = false;
+  const uint8_t *xp = nullptr;
+};
 int launch_linear_codes(const rq_weight *const *w, int count, const void *x, int xtype, int64_t m, const Out *o,
-                        hipStream_t s, WsLease &ws);
+                        hipStream_t s, WsLease &ws, CodesPack *shared = nullptr);
 // The same for Marlin INT4 weights (any k and alignment of x).
 int launch_marlin_codes(const uint32_t *packed, const float *scales, int64_t n, int64_t k, const void *x, int xtype,
                         int64_t m, void *y, int ytype, hipStream_t s, WsLease &ws);

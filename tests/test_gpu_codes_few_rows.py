@@ -73,3 +73,18 @@ def test_rows_that_are_not_finite(dev):
     inf = torch.isinf(want)
     assert bool(inf.any()) and torch.equal(y[2].double()[inf], want[inf])
     assert bool(torch.isnan(y[4]).all())
+
+
+@pytest.mark.parametrize("m", [24, 70, 200])
+@pytest.mark.parametrize("order", [(rq.Q8_0, rq.Q4_K, rq.Q6_K), (rq.Q4_K, rq.Q4_K, rq.Q6_K, rq.Q5_K)])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16])
+def test_formats_that_share_a_pack(dev, m, order, dtype):
+    # runs of several formats on one x, with the sums the K formats need and without
+    k = 4096
+    ws = [rq.QWeight(q, synth.weight_blocks(q, i, 2050, k), 2050, k) for i, q in enumerate(order)]
+    x = torch.from_numpy(synth.activations(m, m, k)).to(dev).to(dtype)
+    for w, y in zip(ws, rq.linear_multi(ws, x)):
+        mag = w.dequantize().double().abs()
+        ref = x.double() @ w.dequantize().double().t()
+        tol = (2.0 ** -15 + EPS[dtype]) * (x.double().abs() @ (mag + (1.26 if w.qtype in (rq.Q4_K, rq.Q5_K) else 0)).t())
+        assert bool(((y.double() - ref).abs() <= tol).all())
