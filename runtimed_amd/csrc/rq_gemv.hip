@@ -17,7 +17,7 @@
 //            lanes, 64 / segment rows per wave (k_gemv_m1);
 //   team     P > 64: a row on a team of ceil(P / 64) waves, one piece per lane
 //            (k_gemv_team);
-//   long     P in 65..128 of a two-run format on n >= 8192: a row on one wave,
+//   long     P in 65..128 of a two-run format on n >= 7168: a row on one wave,
 //            two pieces per lane (k_gemv_long).
 // A lane's pieces keep the same k positions from row to row, so its
 // activations (one row, or two / four row slots for M = 2 / 3) are loaded
@@ -824,9 +824,10 @@ int run_m1(const rq_weight *wt, const void *x, int xtype, const Out &o, hipStrea
   // x 4096 13.1 / 16.4 / 16.6 / 15.4 against 14.1 / 16.9 / 18.8 / 14.7 us, 8192 x
   // 2560 7.9 / 9.7 / 9.7 / 7.9 against 9.1 / 10.6 / 11.8 / 9.0; on 4096 x 4096
   // 8.0 / 9.5 / 10.1 / 8.9 against 6.0 / 6.9 / 7.5 / 6.7, a row a wave and no
-  // second one to overlap).
+  // second one to overlap; between 4096 and 8192 rows a wave takes two at the
+  // cost of 8192 while the team's time falls with n).
   if constexpr (F::RUNS == 2) {
-    if (P > 64 && P <= 128 && wt->n >= 8192) return run_long<F, 2>(wt, x, xtype, o, s);
+    if (P > 64 && P <= 128 && wt->n >= 7168) return run_long<F, 2>(wt, x, xtype, o, s);
   }
   // Other long rows: a team of waves per row.  A lane of the one-wave layout
   // with more pieces holds 128 to 256 activations beside its weight slots and

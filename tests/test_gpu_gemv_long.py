@@ -1,6 +1,6 @@
 """Decode GEMVs on rows of more than 64 pieces (32 elements, 64 for Q6_K) and
 many rows: the team layout on both sides of its rule (two-run formats with at
-most 128 pieces a row and at least 8192 rows walk a row on one wave), with odd
+most 128 pieces a row and at least 7168 rows walk a row on one wave), with odd
 row counts that leave workgroups of unequal length.
 
 Bound per output: f32 activations and exact f32 weights, sums of at most 64
@@ -17,7 +17,7 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("q", [rq.Q4_K, rq.Q5_K, rq.Q6_K, rq.Q8_0, rq.Q4_0, rq.Q5_0])
-@pytest.mark.parametrize("n,k", [(4098, 4224), (8194, 2176), (4097, 4096), (4102, 8320), (4096, 16384)])
+@pytest.mark.parametrize("n,k", [(4098, 4224), (7168, 2176), (8194, 2176), (4097, 4096), (4102, 8320), (4096, 16384)])
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 def test_long_rows_many_rows(dev, q, n, k, dtype):
     print(f"gemv q={q} n={n} k={k} {dtype}", flush=True)
