@@ -98,7 +98,7 @@ __global__ __launch_bounds__(256) void k_fp8_quant_waves(const void *__restrict_
   };
   // Batches of U chunks a lane, their loads issued together; a row of at
   // most one batch stays in registers between the two passes.
-  constexpr int U = WPR == 1 ? 1 : 4;
+  constexpr int U = WPR == 1 ? 1 : F32X ? 4 : 2;
   uint4 buf[U];
   auto load_batch = [&](int64_t c0) {
 #pragma unroll
