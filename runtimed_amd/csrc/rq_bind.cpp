@@ -245,6 +245,19 @@ PyObject *b_kv_dequantize(PyObject *, PyObject *const *a, Py_ssize_t na) {
   END_HANDLE_TH_ERRORS
 }
 
+// dequantize(weight handle, n, k, device index)
+PyObject *b_dequantize(PyObject *, PyObject *const *a, Py_ssize_t na) {
+  HANDLE_TH_ERRORS
+  if (na != 4) Py_RETURN_NONE;
+  const void *h = PyLong_AsVoidPtr(a[0]);
+  const long n = PyLong_AsLong(a[1]), k = PyLong_AsLong(a[2]), dev = PyLong_AsLong(a[3]);
+  if (PyErr_Occurred()) return nullptr;
+  at::Tensor y = at::empty({n, k}, at::TensorOptions().dtype(at::kFloat).device(at::kCUDA, (c10::DeviceIndex)dev));
+  RQ_CALL(rc, rq_dequant_f32(static_cast<const rq_weight *>(h), static_cast<float *>(y.data_ptr()), stream_of(y)));
+  return THPVariable_Wrap(std::move(y));
+  END_HANDLE_TH_ERRORS
+}
+
 // embedding(weight handle, k, device index, u32 ids as a buffer)
 PyObject *b_embedding(PyObject *, PyObject *const *a, Py_ssize_t na) {
   HANDLE_TH_ERRORS
@@ -274,7 +287,8 @@ PyObject *b_embedding(PyObject *, PyObject *const *a, Py_ssize_t na) {
 
 #define RQ_DEF(name) {#name, reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(b_##name)), METH_FASTCALL, nullptr}
 PyMethodDef methods[] = {RQ_DEF(linear),  RQ_DEF(linear_multi),  RQ_DEF(fp8_gemm),  RQ_DEF(marlin),
-                         RQ_DEF(kv_pair), RQ_DEF(kv_dequantize), RQ_DEF(embedding), {nullptr, nullptr, 0, nullptr}};
+                         RQ_DEF(kv_pair), RQ_DEF(kv_dequantize), RQ_DEF(embedding),
+                         RQ_DEF(dequantize), {nullptr, nullptr, 0, nullptr}};
 PyModuleDef module = {PyModuleDef_HEAD_INIT, "_rqc", nullptr, -1, methods, nullptr, nullptr, nullptr, nullptr};
 
 }  // namespace

@@ -170,9 +170,7 @@ class QWeight:
         return {f: getattr(d, f) for f, _ in _Desc._fields_}
 
     def dequantize(self) -> torch.Tensor:
-        out = torch.empty((self.n, self.k), dtype=torch.float32, device=self.device)
-        check(lib().rq_dequant_f32(self._h, _ptr(out), _stream(self.device)))
-        return out
+        return _done((_rqc or _native()).dequantize(self._hv, self.n, self.k, self.device.index))
 
     def embedding(self, ids) -> torch.Tensor:
         """Rows `ids` decoded exactly, f32 [len(ids), k] (embed_layer.rs:16-84)."""
