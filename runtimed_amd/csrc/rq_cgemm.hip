@@ -919,8 +919,8 @@ int go(const WeightSet &set, int64_t tiles, const float *rs, const uint8_t *xp, 
                      xtype, m, k, np, tm, S, part);
   int rc = last_launch("codes gemm");
   if (!rc && S > 1) {
-    hipLaunchKernelGGL((k_cg_sum<D, MI>), dim3((unsigned)(tiles * 8 * MI)), dim3(256), 0, s, set, rs, part, rexp, x, xtype, m,
-                       k, tm, S);
+    hipLaunchKernelGGL((k_cg_sum<D, MI>), dim3((unsigned)(tiles * 8 * MI)), dim3(256), 0, s, set, rs, part, rexp, x,
+                       xtype, m, k, tm, S);
     rc = last_launch("codes gemm sum");
   }
   return rc;

@@ -73,14 +73,8 @@ constexpr int64_t kXldsMaxK = 12288;
 __device__ __forceinline__ int xpad(int e) { return e + 4 * (e >> 6); }
 __host__ __device__ inline size_t xlds_bytes(int64_t k) { return k <= kXldsMaxK ? (size_t)(k + 4 * (k >> 6) + 4) * sizeof(float) : 0; }
 
-__device__ __forceinline__ void stage_x(const void *x, int xtype, int k, float *xs) {
-  for (int e = 4 * (int)threadIdx.x; e < k; e += 4 * (int)blockDim.x)
-    *reinterpret_cast<float4 *>(xs + xpad(e)) = load_x4(x, xtype, e);
-  __syncthreads();
-}
-
-// The same staging split in two, for kernels that issue x's loads before
-// their weight loads: the load counter retires loads in issue order, so a
+// The staging is split in two: kernels issue x's loads before their weight
+// loads, since the load counter retires loads in issue order, so a
 // wait for x loads issued after the weights would hold the staging until the
 // (HBM) weights had landed too.  Thread t loads the 16-byte chunks t,
 // t + blockDim, ... of x (4 f32 or 8 f16/bf16 elements each) with one
@@ -188,13 +182,6 @@ __device__ __forceinline__ void load_run_lds(const float *xs, int e0, float *dst
     dst[4 * j + 2] = a.z;
     dst[4 * j + 3] = a.w;
   }
-}
-
-// Loads run r of piece p: from the LDS copy when there is one (xs != null).
-template <class F>
-__device__ __forceinline__ void load_piece_x(const void *x, int xtype, const float *xs, int p, int r, float *dst) {
-  if (xs) load_run_lds<16>(xs, (int)F::run_off(p, r), dst);
-  else load_run<16>(x, xtype, F::run_off(p, r), dst);
 }
 
 // M = MR (1 or 2), rows of at most 64 pieces: every lane owns one piece
@@ -329,20 +316,19 @@ __global__ __launch_bounds__(256) void k_gemv_set(const WeightSet set, const voi
 // every load is unconditional (rows past n clamp to the slot's own row, just
 // read), so the compiler's waits are exact counts; the last group of D rows
 // refills nothing.  No barriers in the loop: the row total is a DPP sum over
-// the wave.  WPG waves per workgroup share one LDS copy of x.  With XR > 0
-// (XR = 16-byte chunks of x per thread, enough for any k this instance
-// takes) x's loads go out first and the first D rows' weight loads right
-// behind them, so x is staged while the weights are in flight.
+// the wave.  WPG waves per workgroup share one LDS copy of x (XR = 16-byte
+// chunks of x per thread, enough for any k this instance takes): x's loads go
+// out first and the first D rows' weight loads right behind them, so x is
+// staged while the weights are in flight.
 template <class F, int PPL, int WPG>
 constexpr int long_xr() {
-  constexpr int need = (PPL * F::PE + 4 * WPG - 1) / (4 * WPG);  // f32 chunks per thread at k = 64 PPL PE
-  return need <= 4 ? need : 0;
+  return (PPL * F::PE + 4 * WPG - 1) / (4 * WPG);  // f32 chunks per thread at k = 64 PPL PE
 }
 
 template <class F, int PPL, int WPG, int D>
 __global__ __launch_bounds__(64 * WPG) void k_gemv_long(const uint8_t *__restrict__ w,
                                                         const uint8_t *__restrict__ aux, const void *__restrict__ x,
-                                                        int xtype, const Out o, int64_t n, int64_t k, bool xlds) {
+                                                        int xtype, const Out o, int64_t n, int64_t k) {
   constexpr int XR = long_xr<F, PPL, WPG>();
   const int lane = threadIdx.x & 63;
   const int P = (int)(k / F::PE);
@@ -361,19 +347,13 @@ __global__ __launch_bounds__(64 * WPG) void k_gemv_long(const uint8_t *__restric
   const int64_t first = row0 < n ? row0 : n - 1;
 
   extern __shared__ __attribute__((aligned(16))) float xs_dyn[];
-  if constexpr (XR > 0) {  // launched only with the LDS copy of x
-    chunk16 xc[XR];
-    load_x_chunks<XR>(x, xtype, (int)k, xc);
-    __builtin_amdgcn_sched_barrier(0);
+  chunk16 xc[XR];
+  load_x_chunks<XR>(x, xtype, (int)k, xc);
+  __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-    for (int j = 0; j < D; ++j) fill(j, row0 + j * nw, first);
-    __builtin_amdgcn_sched_barrier(0);
-    store_x_chunks<XR>(xtype, (int)k, xc, xs_dyn);
-  } else {
-#pragma unroll
-    for (int j = 0; j < D; ++j) fill(j, row0 + j * nw, first);
-    if (xlds) stage_x(x, xtype, (int)k, xs_dyn);  // uniform: the whole workgroup stages x once
-  }
+  for (int j = 0; j < D; ++j) fill(j, row0 + j * nw, first);
+  __builtin_amdgcn_sched_barrier(0);
+  store_x_chunks<XR>(xtype, (int)k, xc, xs_dyn);
   float xv[PPL][F::RUNS][16];
   float sx[PPL][F::RUNS];
 #pragma unroll
@@ -383,8 +363,7 @@ __global__ __launch_bounds__(64 * WPG) void k_gemv_long(const uint8_t *__restric
     for (int r = 0; r < F::RUNS; ++r) {
       sx[i][r] = 0.0f;
       if (p < P) {
-        if constexpr (XR > 0) load_run_lds<16>(xs_dyn, (int)F::run_off(p, r), xv[i][r]);
-        else load_piece_x<F>(x, xtype, xlds ? xs_dyn : nullptr, p, r, xv[i][r]);
+        load_run_lds<16>(xs_dyn, (int)F::run_off(p, r), xv[i][r]);
 #pragma unroll
         for (int t = 0; t < 16; ++t) sx[i][r] += xv[i][r][t];
       } else {
@@ -677,12 +656,12 @@ int run_long(const rq_weight *wt, const void *x, int xtype, const Out &o, hipStr
   const int64_t waves = wt->n < 256 * 16 ? wt->n : 256 * 16;
   const size_t xb = xlds_bytes(wt->k);
   const unsigned blocks = (unsigned)((waves + 7) / 8);
-  if (long_xr<F, PPL, 8>() > 0 && !xb) return RQ_E_UNSUPPORTED;  // k <= 64 PPL PE always fits the LDS copy
+  if (!xb) return RQ_E_UNSUPPORTED;  // k <= 64 PPL PE always fits the LDS copy
   // Two rows in flight per wave: on Q4_K 14336 x 4096, 10.5 us against
   // 11.9 (three rows) and 13.4 (four), whose registers leave room for one
   // eight-wave workgroup per CU instead of two.
   hipLaunchKernelGGL((k_gemv_long<F, PPL, 8, 2>), dim3(blocks), dim3(512), xb, s, wt->data, wt->data + wt->aux_off,
-                     x, xtype, o, wt->n, wt->k, xb != 0);
+                     x, xtype, o, wt->n, wt->k);
   return hipGetLastError() == hipSuccess ? RQ_OK : set_error(RQ_E_DEVICE, "gemv launch failed");
 }
 
